@@ -236,7 +236,7 @@ __device__ __forceinline__ bool free_stage(gal_state* s, void* ptr, lds_state& L
   }
   if (!(s->flags & kFlagNoPayloadFence) && __ballot(ptr != nullptr)) {
     if (s->num_parts == 1 || __ballot(foreign))
-      utils::fence_release();
+      detail::release_to_device(s);
     else
       detail::release_to_xcd();
   }

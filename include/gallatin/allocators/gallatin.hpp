@@ -55,6 +55,13 @@ using utils::atomic_or;
 using utils::atomic_store;
 using utils::atomic_sub;
 
+constexpr uint32_t kFlushPolls = 4096;     // polls of a flush word before a wave flushes itself
+// Threads of a launch below which every wave flushes by itself: with few waves
+// per XCD the words cost more than the shared write-backs save.  One-word
+// churn of 3 rounds, alone / shared: 1,000 threads 27 / 34 us, 16,000 52 / 56,
+// 32,000 72 / 68, 64,000 122 / 95, 256,000 538 / 422.
+constexpr uint64_t kFlushAlone = 32768;
+
 enum : uint32_t { kPathSlice = 1, kPathBlock = 2, kPathSegment = 3 };
 
 __device__ __forceinline__ bool deterministic(const gal_state* s) {
@@ -110,6 +117,66 @@ __device__ __forceinline__ void add_error(gal_state* s, int kind, uint64_t v = 1
 __device__ __forceinline__ void release_to_xcd() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
+}
+
+// A flush word holds (flushes done << 1) | running.  A caller needs a flush
+// that starts after its call.  Returns kFlushDone when another caller's did,
+// kFlushOwn when this caller is to run one and then add 1 to the word, and
+// kFlushLate when the bounded wait ran out.  Per lane.
+enum : uint32_t { kFlushDone, kFlushOwn, kFlushLate };
+__device__ __forceinline__ uint32_t flush_enter(unsigned long long* word) {
+  unsigned long long w = utils::atomic_or(word, 1ULL);
+  if (!(w & 1)) return kFlushOwn;
+  // the running one may have started before this call: it takes the next
+  const unsigned long long need = (w >> 1) + 2;
+  for (uint32_t polls = 0; polls < kFlushPolls; ++polls) {
+    __builtin_amdgcn_s_sleep(32);
+    w = atomic_load(word);
+    if ((long long)((w >> 1) - need) >= 0) return kFlushDone;
+    if (!(w & 1)) {
+      w = utils::atomic_or(word, 1ULL);
+      if (!(w & 1)) return kFlushOwn;
+    }
+  }
+  return kFlushLate;
+}
+
+// Stores of this wave have left the L2 of its XCD: an agent-scope release.
+// It writes back every dirty line of the XCD's L2, whoever stored it, and
+// write-backs of one L2 run one after another, so the waves of an XCD share
+// them: a write-back that starts after a wave's stores reached the L2 covers
+// them.  The waves of a CU agree on one of them first (its own word), then
+// the CUs of the XCD: one word takes 88 M device atomics/s, and the 512
+// waves of an XCD on one word wait mostly for each other.  2^20 threads of
+// malloc(16), write, read, free on one partition: 262 us with a write-back
+// per wave, 206 us with one word per XCD, 118 us with a word per CU below it
+// (96 us without any release); 1,000,003 threads of ten rounds of the filled
+// churn, 4 pinned blocks per class: 8.5 -> 5.1 ms (4.9 without).
+__device__ __noinline__ void release_shared(gal_state* s) {
+  release_to_xcd();
+  if (wave::is_first()) {
+    unsigned long long* words = s->stats + kStatFlush;
+    const uint32_t cu = __smid() & (kFlushCus - 1);
+    unsigned long long* of_cu = words + kFlushStride * cu;
+    unsigned long long* of_xcd = words + kFlushStride * (kFlushCus + (cu >> 6));
+    const uint32_t c = flush_enter(of_cu);
+    if (c != kFlushDone) {
+      const uint32_t x = flush_enter(of_xcd);
+      if (x != kFlushDone) {
+        utils::fence_release();
+        if (x == kFlushOwn) atomic_add(of_xcd, 1ULL);
+      }
+      if (c == kFlushOwn) atomic_add(of_cu, 1ULL);
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+}
+
+__device__ __forceinline__ void release_to_device(gal_state* s) {
+  if ((uint64_t)gridDim.x * blockDim.x < kFlushAlone)
+    utils::fence_release();
+  else
+    release_shared(s);
 }
 
 // Chunk id field of seg_state: tree 0xFFFF, home 0 (free segment).
@@ -908,7 +975,7 @@ __device__ __forceinline__ void free_impl(gal_state* s, void* ptr) {
   if (!(s->flags & kFlagNoPayloadFence)) {
     // a free away from the segment's home XCD writes this XCD's L2 back
     if (s->num_parts == 1 || __ballot(multi || (slice && seg_home(st) != my_p)))
-      utils::fence_release();
+      release_to_device(s);
     else
       release_to_xcd();
   }

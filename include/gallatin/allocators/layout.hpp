@@ -133,7 +133,13 @@ enum gal_stat {
   // internal, after the reported counters: the last multi-segment search
   // that found no run, as (stat [3] when it started) << 16 | run length
   kStatSegHint = 18,
-  kStatWords = 19
+  // internal: words of release_to_device, each on a cache line of its own:
+  // one per CU (index __smid()), then one per XCD
+  kStatFlush = 32,
+  kFlushStride = 16,
+  kFlushXcds = 16,
+  kFlushCus = 64 * kFlushXcds,
+  kStatWords = kStatFlush + kFlushStride * (kFlushCus + kFlushXcds)
 };
 
 // The instance viewed through the reference's alloc_table accessors

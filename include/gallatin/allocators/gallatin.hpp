@@ -410,12 +410,17 @@ __device__ inline uint64_t get_block(gal_state* s, uint64_t seg, uint32_t t, uin
 
 // gallatin.cuh:1283-1302 submit_segment_for_free: the chunk id is reset
 // before the run goes back to the segment tree, so a concurrent gather can
-// never find the head still marked.
+// never find the head still marked.  Every active lane gives back its own
+// run of n segments (lanes with n = 0 none): the chain of dependent accesses
+// is one run's, where run after run a wave of the 64 KiB - 2 GiB mix took
+// about 4 us for each (571 requests checked and freed: 241 -> 44 us).
 __device__ __noinline__ void free_segments(gal_state* s, uint64_t seg, uint64_t n) {
-  clear_chunk_id(s, seg);
+  if (n) clear_chunk_id(s, seg);
   utils::fence_release();
-  veb::return_multiple(s->seg_tree, seg, n);
-  add_stat(s, kStatSegmentsReleased, n);
+  if (n) veb::return_multiple(s->seg_tree, seg, n);
+  uint32_t below, total;
+  wave::group_scan((uint32_t)n, __ballot(1), below, total);
+  if (wave::is_first()) add_stat(s, kStatSegmentsReleased, total);
 }
 
 // shared_block_storage.cuh:119-134 get_valid_block_index + get_my_block for
@@ -979,13 +984,7 @@ __device__ __forceinline__ void free_impl(gal_state* s, void* ptr) {
     else
       release_to_xcd();
   }
-  // multi-segment frees one at a time in lane order
-  for (uint64_t m = __ballot(multi); m; m &= m - 1) {
-    const int l = wave::first(m);
-    const uint64_t sg = wave::readlane(seg, l);
-    const uint32_t tl = wave::readlane(t, l);
-    if (wave::is_first()) free_segments(s, sg, tl - T - 1);
-  }
+  if (__ballot(multi)) free_segments(s, seg, multi ? t - T - 1 : 0);
   const uint64_t sm = __ballot(slice);
   if (!sm) return;
   uint32_t blk = 0;
@@ -1013,12 +1012,18 @@ __device__ __forceinline__ void free_impl(gal_state* s, void* ptr) {
     const uint32_t old = atomic_add(&block_at(s, blk)->free_counter, k);
     completes = old + k == kSlicesPerBlock;
   }
-  for (uint64_t m = __ballot(completes); m; m &= m - 1) {
-    const uint32_t b = wave::readlane(blk, wave::first(m));
-    if (wave::is_first()) {
-      atomic_exch(&block_at(s, b)->free_counter, 0u);
-      free_block(s, b, my_p);
+  // completed blocks go back to their segments all at once; in the
+  // deterministic mode in lane order, which sets the order of the rings
+  if (det) {
+    for (uint64_t m = __ballot(completes); m; m &= m - 1) {
+      if ((int)lane == wave::first(m)) {
+        atomic_exch(&block_at(s, blk)->free_counter, 0u);
+        free_block(s, blk, my_p);
+      }
     }
+  } else if (completes) {
+    atomic_exch(&block_at(s, blk)->free_counter, 0u);
+    free_block(s, blk, my_p);
   }
 }
 

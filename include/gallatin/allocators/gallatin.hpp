@@ -56,8 +56,9 @@ using utils::atomic_store;
 using utils::atomic_sub;
 
 constexpr uint32_t kFlushPolls = 4096;     // polls of a flush word before a wave flushes itself
-// Threads of a launch below which every wave flushes by itself: with few waves
-// per XCD the words cost more than the shared write-backs save.  One-word
+// Threads of a launch below which every wave flushes by itself (and below 128
+// workgroups of any size): with few waves per XCD the words cost more than the
+// shared write-backs save.  One-word
 // churn of 3 rounds, alone / shared: 1,000 threads 27 / 34 us, 16,000 52 / 56,
 // 32,000 72 / 68, 64,000 122 / 95, 256,000 538 / 422.
 constexpr uint64_t kFlushAlone = 32768;
@@ -154,6 +155,10 @@ __device__ __forceinline__ uint32_t flush_enter(unsigned long long* word) {
 // churn, 4 pinned blocks per class: 8.5 -> 5.1 ms (4.9 without).
 __device__ __noinline__ void release_shared(gal_state* s) {
   release_to_xcd();
+  if ((uint64_t)gridDim.x * blockDim.x < kFlushAlone) {
+    utils::fence_release();
+    return;
+  }
   if (wave::is_first()) {
     unsigned long long* words = s->stats + kStatFlush;
     const uint32_t cu = __smid() & (kFlushCus - 1);
@@ -172,8 +177,10 @@ __device__ __noinline__ void release_shared(gal_state* s) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
 }
 
+// The workgroup count alone settles it for a small launch: multiplying out
+// the threads here cost such a launch 0.15 us per free.
 __device__ __forceinline__ void release_to_device(gal_state* s) {
-  if ((uint64_t)gridDim.x * blockDim.x < kFlushAlone)
+  if (gridDim.x < kFlushAlone / 256)
     utils::fence_release();
   else
     release_shared(s);

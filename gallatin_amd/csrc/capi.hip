@@ -83,7 +83,10 @@ __global__ void k_boot(gal_state* s) {
   for (uint32_t t = 0; t < s->num_trees; ++t) {
     const uint32_t per = s->slot_count[t] / s->num_parts;
     for (uint32_t i = 0; i < s->slot_count[t]; ++i) {
-      const uint32_t blk = detail::request_new_block(s, t, i / per, true, s->lim_request);
+      bool emptied;
+      const uint32_t blk = wave::readfirst(detail::request_new_blocks(
+          s, t, i / per, true, s->lim_request, wave::is_first(), emptied));
+      if (__ballot(emptied)) detail::prefetch_segment(s, t, i / per);
       if (blk == kNullBlock) {
         if (wave::is_first()) utils::atomic_store(&s->stats[kStatBootFailed], 1ULL);
         return;

@@ -420,7 +420,7 @@ __device__ inline uint64_t get_block(gal_state* s, uint64_t seg, uint32_t t, uin
 // never find the head still marked.  Every active lane gives back its own
 // run of n segments (lanes with n = 0 none): the chain of dependent accesses
 // is one run's, where run after run a wave of the 64 KiB - 2 GiB mix took
-// about 4 us for each (571 requests checked and freed: 241 -> 44 us).
+// about 4 us for each (571 requests checked and freed: 241 -> 27 us).
 __device__ __noinline__ void free_segments(gal_state* s, uint64_t seg, uint64_t n) {
   if (n) clear_chunk_id(s, seg);
   utils::fence_release();
@@ -532,6 +532,50 @@ __device__ inline uint64_t gather_new_segment(gal_state* s, uint32_t t, uint32_t
   return seg;
 }
 
+// gather_new_segment for up to `most` segments at once, for a class of few
+// blocks per segment: the segments come from one word of the segment tree and
+// each lane sets one up.  Returns the r-th segment on the r-th active lane,
+// kFail on the lanes past them.
+__device__ inline uint64_t gather_new_segments(gal_state* s, uint32_t t, uint32_t p,
+                                               uint32_t most) {
+  uint64_t w = 0;
+  uint64_t m = veb::take_some(s->seg_tree, most, w);
+  const uint32_t rank = wave::count(wave::active() & wave::lanes_below());
+  const bool mine = rank < wave::count(m);
+  for (uint32_t k = 0; mine && k < rank; ++k) m &= m - 1;
+  const uint64_t seg = mine ? (w << 6) + (uint64_t)wave::first(m) : kFail;
+  bool ok = false;
+  if (mine) {
+    uint64_t cur = atomic_load(&s->seg_state[seg]);
+    for (int g = 0; g < 4096 && (cur & 0xFFFF) == kFreeTree; ++g) {
+      const uint64_t seen =
+          atomic_cas(&s->seg_state[seg], cur, (cur & ~kSegIdMask) | seg_id(t, p));
+      ok = seen == cur;
+      if (ok) break;
+      cur = seen;
+    }
+    if (ok) {
+      const uint64_t nb = nb_of(s, t);
+      for (uint64_t i = 0; i < nb; ++i)
+        atomic_store(&s->ring[(seg << s->bps_shift) + i], kNullBlock);
+      gal_seg_queue* q = &s->seg_queue[seg];
+      atomic_store(&q->q_malloc, 0u);
+      atomic_store(&q->q_free, 0u);
+      const uint64_t gen = (atomic_load(&q->q_done) >> kDoneGenShift) + 1;
+      atomic_store(&q->q_done, gen << kDoneGenShift);
+    } else {
+      add_error(s, kStatErrSetup);
+    }
+  }
+  release_to_xcd();
+  if (ok) {
+    atomic_add(&s->seg_state[seg], nb_of(s, t) << 32);  // active -1 -> nb-1
+    add_stat(s, kStatSegmentsSetUp, 1);
+    veb::insert(class_tree(s, t, p), seg);
+  }
+  return ok ? seg : kFail;
+}
+
 // Segment of class t (partition p) to take a block from: smallest id in
 // deterministic mode (find_first_valid_index, veb.cuh:940-944), else from a
 // hashed start (find_random_valid_index, veb.cuh:946-977) wrapping to 0.
@@ -547,18 +591,31 @@ __device__ inline uint64_t find_segment(gal_state* s, uint32_t t, uint32_t p, bo
   return x;
 }
 
-// gallatin.cuh:1525-1631 request_new_block_from_tree.  With no segment in
-// the class tree and none free it polls (up to `polls` times, lim_request
-// for a first request): frees in flight on other waves return segments
-// within microseconds.
-__device__ inline uint32_t request_new_block(gal_state* s, uint32_t t, uint32_t p,
-                                             bool det, uint32_t polls) {
+// gallatin.cuh:1525-1631 request_new_block_from_tree, for every lane with
+// `want` at once: each gets a block id of class t, or kNullBlock.  With no
+// segment in the class tree and none free it polls (up to `polls` times,
+// lim_request for a first request): frees in flight on other waves return
+// segments within microseconds.  The lanes share every search and take
+// their blocks side by side; run one request after another, each cost a
+// chain of about 5 dependent atomics (1.1 us each) and a search (571
+// requests of 64 KiB - 2 GiB: 316 us one after another, 178 us together).
+// `emptied`: this lane took its segment's last block, and the caller runs
+// prefetch_segment once it has passed the block on.
+__device__ inline uint32_t request_new_blocks(gal_state* s, uint32_t t, uint32_t p, bool det,
+                                              uint32_t polls, bool want, bool& emptied) {
   int attempts = 0;
   uint64_t released = 0;  // segments given back so far, at the last check
   const uint32_t lk = tree_lock(s, t, p);
+  uint32_t blk = kNullBlock;
+  emptied = false;
   for (uint32_t spins = 0; attempts < (int)polls && spins < kSpinCap;
        ++spins) {
+    const uint64_t pend = __ballot(want && blk == kNullBlock);
+    if (!pend) break;
+    const uint32_t k = wave::count(pend);
+    const uint32_t rank = wave::count(pend & wave::lanes_below());
     uint64_t seg = find_segment(s, t, p, det);
+    bool fresh = false;
     if (seg == kFail) {
       if (veb::looks_empty(s->seg_tree)) {
         // nothing free: poll without taking the class lock, whose release
@@ -580,34 +637,58 @@ __device__ inline uint32_t request_new_block(gal_state* s, uint32_t t, uint32_t 
         utils::backoff();
         continue;
       }
-      seg = gather_new_segment(s, t, p);
+      const uint64_t nb = nb_of(s, t);
+      if (!det && k > nb) {
+        // the pending lanes take the segments in turn, nb lanes each
+        const uint64_t got = gather_new_segments(s, t, p, (uint32_t)((k + nb - 1) / nb));
+        const uint64_t have = __ballot(got != kFail);
+        const uint32_t nth = (uint32_t)(rank / nb);
+        uint64_t m = have;
+        for (uint32_t j = 0; m && j < nth; ++j) m &= m - 1;
+        const uint64_t of = wave::fetch(got, m ? wave::first(m) : 0);
+        seg = have ? (m ? of : kFail) : kNoSegment;
+        fresh = true;
+      } else {
+        seg = gather_new_segment(s, t, p);
+      }
       unlock(s, lk);
-      if (seg == kFail || seg == kNoSegment) {
+      if (!__ballot(seg != kFail && seg != kNoSegment)) {
         ++attempts;
         if (seg == kNoSegment) utils::backoff();
         continue;
       }
     }
-    uint64_t got = kNullBlock;
-    if (wave::is_first()) got = get_block(s, seg, t, p, spins > 0);
-    got = wave::readfirst(got);
-    if (got >> 32) {
-      // segment fully handed out: detach it and prefetch the next one
-      // (gallatin.cuh:1611-1614).  With XCD partitions a segment whose
-      // last block came back on a foreign XCD stays formatted in its home's
-      // class tree, so the prefetch waits until that tree is empty: taking a
-      // fresh segment for every reused one would format segments without
-      // bound (a 1-block class does it on every block).
-      if (wave::is_first()) veb::remove(class_tree(s, t, p), seg);
-      if ((s->num_parts == 1 || veb::looks_empty(class_tree(s, t, p))) && try_lock(s, lk)) {
-        gather_new_segment(s, t, p);
-        unlock(s, lk);
+    // of several lanes on one segment, those past its free blocks would only
+    // subtract and add back
+    bool take = want && blk == kNullBlock && seg < kNoSegment;
+    if (k > 1 && !fresh && take) {
+      const int32_t active = (int32_t)(atomic_load(&s->seg_state[seg]) >> 32);
+      take = (int64_t)rank <= (int64_t)active;
+    }
+    if (take) {
+      const uint64_t got = get_block(s, seg, t, p, spins > 0);
+      blk = (uint32_t)got;
+      if (got >> 32) {
+        veb::remove(class_tree(s, t, p), seg);
+        emptied = true;
       }
     }
-    const uint32_t blk = (uint32_t)got;
-    if (blk != kNullBlock) return blk;
   }
-  return kNullBlock;
+  return blk;
+}
+
+// After a segment was handed out in full (and detached), take the next one
+// for its class (gallatin.cuh:1611-1614).  With XCD partitions a segment whose
+// last block came back on a foreign XCD stays formatted in its home's
+// class tree, so the prefetch waits until that tree is empty: taking a
+// fresh segment for every reused one would format segments without
+// bound (a 1-block class does it on every block).
+__device__ inline void prefetch_segment(gal_state* s, uint32_t t, uint32_t p) {
+  const uint32_t lk = tree_lock(s, t, p);
+  if ((s->num_parts == 1 || veb::looks_empty(class_tree(s, t, p))) && try_lock(s, lk)) {
+    gather_new_segment(s, t, p);
+    unlock(s, lk);
+  }
 }
 
 // Refill an empty pinned slot of class t (wave op).  Returns the block now
@@ -623,12 +704,15 @@ __device__ __noinline__ uint32_t refill_slot(gal_state* s, uint32_t t, uint32_t 
   if (wave::is_first()) cur = atomic_cas(sp, kNullBlock, kRefilling);
   cur = wave::readfirst(cur);
   if (cur != kNullBlock) return cur;  // a block, or another wave's refill
-  const uint32_t nb = request_new_block(s, t, p, det, s->lim_request);
+  bool emptied;
+  const uint32_t nb =
+      request_new_blocks(s, t, p, det, s->lim_request, wave::is_first(), emptied);
   if (wave::is_first()) {
     atomic_exch(sp, nb);  // the block, or empty again
     if (nb != kNullBlock) add_stat(s, kStatRefills, 1);
   }
-  return nb;
+  if (__ballot(emptied)) prefetch_segment(s, t, p);
+  return wave::readfirst(nb);
 }
 
 // gallatin.cuh:1083-1138 replace_block.  The detached slot holds kRefilling
@@ -648,8 +732,13 @@ __device__ __noinline__ void replace_block(gal_state* s, uint32_t t, uint32_t p,
       retire_block(s, blk, p);
   }
   if (wave::readfirst(seen) != blk) return;
-  const uint32_t nb = request_new_block(s, t, p, det, s->lim_request);
+  bool emptied;
+  const uint32_t nb =
+      request_new_blocks(s, t, p, det, s->lim_request, wave::is_first(), emptied);
   if (wave::is_first()) atomic_exch(sp, nb);
+  // the waves waiting for the slot have their block; the set-up of the next
+  // segment takes a lock and about 10 us
+  if (__ballot(emptied)) prefetch_segment(s, t, p);
 }
 
 // Slice phase of malloc: gallatin.cuh:865-1078 malloc_slice_allocation for
@@ -758,29 +847,49 @@ __device__ __forceinline__ void malloc_slices(gal_state* s, bool want, uint32_t 
 
 // gallatin.cuh:828-861 malloc_block_allocation + block.cuh:288-340
 // malloc_fill_block, retried as gallatin.cuh:1226-1231 while blocks are
-// handed out but lost to a concurrent claim.  Byte offset.
-__device__ __noinline__ uint64_t malloc_block_path(gal_state* s, uint32_t bt, uint32_t p,
-                                                   bool det, uint32_t polls) {
-  for (uint32_t attempt = 0; attempt < s->lim_block; ++attempt) {
-    const uint32_t blk = request_new_block(s, bt, p, det, polls);
-    if (blk == kNullBlock) return kFail;
-    uint32_t res = 0;
-    if (wave::is_first()) {
-      const uint32_t merged = atomic_add(&block_at(s, blk)->malloc_counter, 4096u);
-      const uint32_t oldc = merged & kCountMask;
-      if ((merged >> kTreeShift) != block_tag(bt, p)) {  // check_valid -> trap
-        add_error(s, kStatErrTag);
-      } else {
-        atomic_add(&block_at(s, blk)->free_counter, 4095u - oldc);
-        if (oldc != 0)
-          block_release(s, blk, 1, p);
-        else
-          res = 1;
+// handed out but lost to a concurrent claim, for the lanes with `want` (a
+// block of class bt each).  The lanes of a class are served together, in the
+// deterministic mode one after another.  Once a lane has polled out its
+// attempts with no segment to be had, the later classes try once each (any
+// class tree may still hold a segment with a free block) instead of polling
+// the same empty pool again.  Only the deterministic mode, which replays the
+// reference's steps, prefetches the next segment here: nothing waits for one,
+// and the next request of the class takes as many as it needs.  Byte offset
+// per lane, kFail on a miss.
+__device__ __noinline__ uint64_t malloc_blocks(gal_state* s, bool want, uint32_t bt, uint32_t p,
+                                               bool det) {
+  uint64_t out = kFail;
+  uint32_t polls = s->lim_request;
+  for (uint64_t todo = __ballot(want); todo;) {
+    const int l = wave::first(todo);
+    const uint32_t t = wave::readlane(bt, l);
+    const uint64_t grp = det ? 1ULL << l : todo & __ballot(want && bt == t);
+    todo &= ~grp;
+    bool open = (grp >> wave::lane()) & 1;
+    for (uint32_t attempt = 0; attempt < s->lim_block && __ballot(open); ++attempt) {
+      bool emptied;
+      const uint32_t blk = request_new_blocks(s, t, p, det, polls, open, emptied);
+      if (__ballot(open && blk == kNullBlock)) polls = 1;
+      open = open && blk != kNullBlock;
+      if (open) {
+        const uint32_t merged = atomic_add(&block_at(s, blk)->malloc_counter, 4096u);
+        const uint32_t oldc = merged & kCountMask;
+        if ((merged >> kTreeShift) != block_tag(t, p)) {  // check_valid -> trap
+          add_error(s, kStatErrTag);
+        } else {
+          atomic_add(&block_at(s, blk)->free_counter, 4095u - oldc);
+          if (oldc != 0) {
+            block_release(s, blk, 1, p);
+          } else {
+            out = offset_to_bytes(s, (uint64_t)blk << 12, t);
+            open = false;
+          }
+        }
       }
+      if (det && __ballot(emptied)) prefetch_segment(s, t, p);
     }
-    if (wave::readfirst(res)) return offset_to_bytes(s, (uint64_t)blk << 12, bt);
   }
-  return kFail;
+  return out;
 }
 
 // set_tree_id (memory_table.cuh:823-828) for the head of an n-segment run:
@@ -936,16 +1045,9 @@ __device__ __forceinline__ void* malloc_impl(gal_state* s, uint64_t size, bool w
     malloc_slices(s, path == kPathSlice, t, cnt, p, off);
     if (off != kFail) bytes = offset_to_bytes(s, off, t);
   }
-  // The block requests of a wave run one after another.  Once one of them
-  // has polled out its attempts with no segment to be had, the rest try
-  // once each (any class tree may still hold a segment with a free block)
-  // instead of polling the same empty pool again.
-  uint32_t polls = s->lim_request;
-  for (uint64_t m = __ballot(path == kPathBlock); m; m &= m - 1) {
-    const int l = wave::first(m);
-    const uint64_t r = malloc_block_path(s, wave::readlane(t, l), p, det, polls);
-    if (r == kFail) polls = 1;
-    if ((int)lane == l) bytes = r;
+  if (__ballot(path == kPathBlock)) {
+    const uint64_t r = malloc_blocks(s, path == kPathBlock, t, p, det);
+    if (path == kPathBlock) bytes = r;
   }
   if (__ballot(path == kPathSegment)) {
     const uint64_t r = malloc_segments(s, path == kPathSegment, nseg, det);

@@ -159,6 +159,29 @@ __device__ inline uint64_t take_first(const gal_tree& t) {
   return kFail;
 }
 
+// Takes up to `most` available indices of one word, the lowest ones of the
+// first word that has any, with one atomic.  Returns their mask and in `w`
+// the word's index; 0 when the tree shows none.  Wave-cooperative.
+__device__ inline uint64_t take_some(const gal_tree& t, uint32_t most, uint64_t& w) {
+  for (int attempt = 0; attempt < 15; ++attempt) {
+    const uint64_t x = find_ge(t, 0);
+    if (x == kFail) return 0;
+    w = x >> 6;
+    uint64_t got = 0;
+    if (wave::is_first()) {
+      uint64_t* p = word(t, t.num_layers - 1, w);
+      uint64_t v = atomic_load(p), m = 0;
+      for (uint32_t k = 0; v && k < most; ++k, v &= v - 1) m |= v & -v;
+      const uint64_t old = m ? atomic_and(p, ~m) : 0;
+      got = old & m;
+      if (got && (old & ~m) == 0) sync_up(t, t.num_layers - 1, w);
+    }
+    got = wave::readfirst(got);
+    if (got) return got;
+  }
+  return 0;
+}
+
 // Contiguous run of n available indices, claimed atomically; returns the
 // lowest index or kFail.  Candidate runs end at the top of a word's
 // trailing-ones run and extend downward (veb.cuh:323-452); the candidate of

@@ -482,10 +482,14 @@ int gal_run_big(gal_allocator* a, uint64_t seed, uint32_t step, uint64_t n_small
   if (n == 0) return GAL_OK;
   if (n > (1ULL << 32)) return fail(GAL_ERR_INVALID, "at most 2^32 requests per step");
   hipStream_t st = (hipStream_t)stream;
-  k_big_malloc<<<grid_for(n, 256), 256, 0, st>>>(a->dev, seed, step, n, n_small, ptrs, ctr);
+  // One wave per workgroup: consecutive workgroups go to different XCDs, so
+  // the waves of a step work on different partitions' class locks and trees.
+  // With four waves per workgroup the waves of one XCD queued on each other:
+  // 571 requests took 178 us to allocate against 110.
+  k_big_malloc<<<grid_for(n, 64), 64, 0, st>>>(a->dev, seed, step, n, n_small, ptrs, ctr);
   int rc = launch_status("big_malloc");
   if (rc != GAL_OK) return rc;
-  k_big_free<<<grid_for(n, 256), 256, 0, st>>>(a->dev, seed, step, n, ptrs, ctr);
+  k_big_free<<<grid_for(n, 64), 64, 0, st>>>(a->dev, seed, step, n, ptrs, ctr);
   return launch_status("big_free");
 }
 

@@ -1027,7 +1027,7 @@ __global__ void k_serve_table(table_large* t, uint64_t seed, uint32_t step, uint
   const uint64_t r = mix3(seed ^ 0x5eedULL, step, i);
   const uint64_t key = (r & ((1ULL << 28) - 1)) + 1;
   const bool ins = (r >> 40) % 10 < 7;
-  const bool ok = ins ? t->insert(key, r) : t->remove(key);
+  const bool ok = t->update(ins, key, r);
   count_wave(&ctr[kSrvHtInserted], ins && ok);
   count_wave(&ctr[kSrvHtFailed], ins && !ok);
   count_wave(&ctr[kSrvHtRemoved], !ins && ok);

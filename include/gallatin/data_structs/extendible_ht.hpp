@@ -14,8 +14,8 @@
 // creation.
 //
 // Writes (insert, remove) lock the owner bucket, check that it still owns
-// the key and work under the lock.  The lock bit and the depth share one
-// word, so the atomic that takes the lock also returns the depth.  A full
+// the key and work under the lock.  The lock bit, the depth and the home
+// share one word, so the atomic that takes the lock also returns both.  A full
 // bucket is split: a new bucket with home h(b) + 2^d(b) and depth d(b) + 1
 // receives the keys whose bit d(b) is set, is published in the directory,
 // then the old bucket's depth is raised and the moved keys are cleared from
@@ -27,6 +27,16 @@
 // reused).  Every bucket word is read and written with device-coherent
 // atomics; a value is written before its key and a moved key before the new
 // bucket is published.  Lock attempts per operation are bounded.
+//
+// What bounds it: coherent requests.  A lane that reads its own bucket's 17
+// words one by one issues 17 of them per key, and the device serves 250 G/s of
+// such scattered requests.  So a bucket of 15 pairs starts with one 128-byte
+// line, the control word and the keys, and the lanes of a whole wave read the
+// lines together: eight lanes per bucket, 16 bytes each, so that a line is
+// one request.  The first look at the directory goes through the XCD's
+// caches (see owner).  2^20 operations on a table of 2^21 keys: query
+// 114 -> 76 us, insert 215 -> 157 us, remove 183 -> 99 us (the last two are then
+// bound by their lock atomics and stores, 4 and 3 an operation at 26 G/s).
 //
 // Differences from the reference: insert of a present key replaces its
 // value; remove() exists (the reference has none, so its behaviour is not
@@ -98,13 +108,16 @@ struct extendible_hash_table {
   static constexpr uint64_t min_items = 1ULL << min_bits;
   static constexpr uint64_t max_items = 1ULL << max_bits;
   static constexpr uint32_t kTries = 1u << 22;  // lock attempts per operation
+  static constexpr uint32_t kSameBucket = 6;    // lost lock attempts before looking up again
+  static constexpr uint32_t kTogether = 8;      // lanes from which a wave reads lines together
 
   struct bucket {
-    uint64_t ctl;  // (depth << 32) | lock bit
-    uint64_t home;
+    uint64_t ctl;  // (home << 8) | (depth << 1) | lock bit
     uint64_t keys[items_per_bucket];
     uint64_t vals[items_per_bucket];
   };
+  // the control word and the keys fill one 128-byte line of an aligned bucket
+  static constexpr bool kLine = items_per_bucket == 15;
 
   bucket** directory;  // max_items entries
   uint64_t level;      // deepest bucket depth
@@ -171,8 +184,7 @@ struct extendible_hash_table {
     if (!b) return nullptr;
     // device-coherent stores: another XCD may read the bucket as soon as
     // it is published
-    gallatin::utils::atomic_store(&b->ctl, (uint64_t)depth << 32);
-    gallatin::utils::atomic_store(&b->home, home);
+    gallatin::utils::atomic_store(&b->ctl, ctl_of(home, depth));
     for (int i = 0; i < items_per_bucket; ++i)
       gallatin::utils::atomic_store(&b->keys[i], (uint64_t)defaultKey);
     return b;
@@ -225,22 +237,109 @@ struct extendible_hash_table {
 
   __device__ uint64_t hash(Key k) const { return hashers::MurmurHash64A_u64((uint64_t)k, seed); }
 
-  // All keys of a bucket (and its home) are loaded first, so the loads are
-  // in flight together, then compared: the slot holding `key` or -1, and
-  // the first free slot or -1.
-  __device__ uint64_t scan(bucket* b, uint64_t key, int& match, int& empty) {
-    uint64_t k[items_per_bucket];
-    const uint64_t home = ld(&b->home);
-#pragma unroll
-    for (int s = 0; s < items_per_bucket; ++s) k[s] = ld(&b->keys[s]);
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+  // Eight device-coherent 16-byte loads in flight together (each 8-byte half
+  // is read whole).  The wait is part of the block, so no output register is
+  // reused while its load is still on the way.
+  static __device__ __forceinline__ void load8(const uint64_t (&a)[8], u32x4 (&w)[8]) {
+    asm volatile(
+        "global_load_dwordx4 %0, %8, off sc1\n\t"
+        "global_load_dwordx4 %1, %9, off sc1\n\t"
+        "global_load_dwordx4 %2, %10, off sc1\n\t"
+        "global_load_dwordx4 %3, %11, off sc1\n\t"
+        "global_load_dwordx4 %4, %12, off sc1\n\t"
+        "global_load_dwordx4 %5, %13, off sc1\n\t"
+        "global_load_dwordx4 %6, %14, off sc1\n\t"
+        "global_load_dwordx4 %7, %15, off sc1\n\t"
+        "s_waitcnt vmcnt(0)"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]),
+          "=&v"(w[6]), "=&v"(w[7])
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7])
+        : "memory");
+  }
+  static __device__ __forceinline__ uint64_t lo(u32x4 v) {
+    return (uint64_t)v.x | (uint64_t)v.y << 32;
+  }
+  static __device__ __forceinline__ uint64_t hi(u32x4 v) {
+    return (uint64_t)v.z | (uint64_t)v.w << 32;
+  }
+  static __device__ __forceinline__ bool is_free(uint64_t k) {
+    return k == (uint64_t)defaultKey || k == (uint64_t)tombstoneKey;
+  }
+
+  // Bucket b's control word, the slot holding `key` or -1, and the first free
+  // slot or -1, for every lane with `on` (the others get nothing of use).  All
+  // words are loaded first, so the loads are in flight together, then
+  // compared.
+  __device__ void scan(bool on, bucket* b, uint64_t key, uint64_t& ctl, int& match, int& empty) {
+    const uint64_t todo = __ballot(on);
     match = -1;
     empty = -1;
+    ctl = 0;
+    if (!todo) return;
+    if constexpr (kLine) {
+      uint64_t a[8];
+      u32x4 w[8];
+      if (__ballot(1) == ~0ULL && gallatin::wave::count(todo) >= kTogether) {
+        // round r serves lanes 8r .. 8r + 7: lane l reads the l % 8-th 16
+        // bytes of the bucket of lane 8r + l / 8
+        const uint32_t lane = gallatin::wave::lane();
+        const int any = gallatin::wave::first(todo);  // stands in for lanes that ask nothing
+        const uint64_t mine = reinterpret_cast<uint64_t>(b);
+        const uint64_t at = on ? mine : gallatin::wave::readlane(mine, any);
 #pragma unroll
-    for (int s = items_per_bucket - 1; s >= 0; --s) {
-      if (k[s] == key) match = s;
-      if (k[s] == (uint64_t)defaultKey || k[s] == (uint64_t)tombstoneKey) empty = s;
+        for (int r = 0; r < 8; ++r)
+          a[r] = gallatin::wave::fetch(at, 8 * r + (int)(lane >> 3)) + 16 * (lane & 7);
+        load8(a, w);
+        uint64_t m0 = 0, m1 = 0, e0 = 0, e1 = 0;  // this lane's round's answers
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const uint64_t k = gallatin::wave::fetch(key, 8 * r + (int)(lane >> 3));
+          const uint64_t x0 = lo(w[r]), x1 = hi(w[r]);
+          const bool first = (lane & 7) == 0;  // x0 is the control word
+          const uint64_t q0 = __ballot(!first && x0 == k), q1 = __ballot(x1 == k);
+          const uint64_t f0 = __ballot(!first && is_free(x0)), f1 = __ballot(is_free(x1));
+          const uint64_t c = gallatin::wave::fetch(x0, (int)(8 * (lane & 7)));
+          const bool me = (int)(lane >> 3) == r;
+          m0 = me ? q0 : m0;
+          m1 = me ? q1 : m1;
+          e0 = me ? f0 : e0;
+          e1 = me ? f1 : e1;
+          ctl = me ? c : ctl;
+        }
+        // byte l % 8: bit j of m0 is slot 2j - 1, of m1 slot 2j
+        const uint32_t sh = 8 * (lane & 7);
+        const uint32_t q0 = (uint32_t)(m0 >> sh) & 255u, q1 = (uint32_t)(m1 >> sh) & 255u;
+        const uint32_t f0 = (uint32_t)(e0 >> sh) & 255u, f1 = (uint32_t)(e1 >> sh) & 255u;
+        if (q0 | q1) match = q0 ? 2 * __builtin_ctz(q0) - 1 : 2 * __builtin_ctz(q1);
+        const int s0 = f0 ? 2 * __builtin_ctz(f0) - 1 : 15, s1 = f1 ? 2 * __builtin_ctz(f1) : 15;
+        const int s = s0 < s1 ? s0 : s1;
+        if (s < 15) empty = s;
+      } else if (on) {  // few, or some lanes are elsewhere: each its own bucket's line
+#pragma unroll
+        for (int r = 0; r < 8; ++r) a[r] = reinterpret_cast<uint64_t>(b) + 16 * r;
+        load8(a, w);
+        ctl = lo(w[0]);
+#pragma unroll
+        for (int r = 7; r >= 0; --r) {
+          if (hi(w[r]) == key) match = 2 * r;
+          if (is_free(hi(w[r]))) empty = 2 * r;
+          if (r > 0 && lo(w[r]) == key) match = 2 * r - 1;
+          if (r > 0 && is_free(lo(w[r]))) empty = 2 * r - 1;
+        }
+      }
+    } else if (on) {
+      uint64_t k[items_per_bucket];
+      ctl = ld(&b->ctl);
+#pragma unroll
+      for (int s = 0; s < items_per_bucket; ++s) k[s] = ld(&b->keys[s]);
+#pragma unroll
+      for (int s = items_per_bucket - 1; s >= 0; --s) {
+        if (k[s] == key) match = s;
+        if (is_free(k[s])) empty = s;
+      }
     }
-    return home;
   }
 
   // The bucket owning hash h: the entry of its low `level` bits, or of
@@ -248,11 +347,12 @@ struct extendible_hash_table {
   // set, so the deepest one present among the loaded depths is the owner
   // (or a bucket being split, which the callers' home check rejects).
   //
-  // `fresh` = false reads `level` through the cache: it may be behind, which
-  // only leads to an ancestor of the owner, and every caller checks the
+  // `fresh` = false reads `level` and the entries through the caches: they
+  // may be behind, and since the level only grows and entries are only ever
+  // set that only leads to an ancestor of the owner; every caller checks the
   // bucket's home against its depth and looks again (with fresh = true).
-  // Every operation reads `level`, and device-coherent reads of one word
-  // from the whole device queue at one memory channel.
+  // Device-coherent reads of one word from the whole device queue at one
+  // memory channel, and scattered ones run at half the rate of cached ones.
   static constexpr int kOwnerFan = 4;
   __device__ bucket* owner(uint64_t h, bool fresh) {
     uint64_t top = fresh ? ld(&level) : ld_cached(&level);
@@ -261,7 +361,8 @@ struct extendible_hash_table {
 #pragma unroll
       for (int j = 0; j < kOwnerFan; ++j) {
         const uint64_t d = top >= min_bits + j ? top - j : min_bits;
-        e[j] = ld(reinterpret_cast<uint64_t*>(&directory[h & mask(d)]));
+        const uint64_t* at = reinterpret_cast<const uint64_t*>(&directory[h & mask(d)]);
+        e[j] = fresh ? ld(at) : ld_cached(at);
       }
 #pragma unroll
       for (int j = 0; j < kOwnerFan; ++j)
@@ -272,23 +373,30 @@ struct extendible_hash_table {
   }
 
   static __device__ __forceinline__ uint32_t depth_of(uint64_t ctl) {
-    return (uint32_t)(ctl >> 32);
+    return (uint32_t)(ctl >> 1) & 127u;
+  }
+  static __device__ __forceinline__ uint64_t home_of(uint64_t ctl) { return ctl >> 8; }
+  static __device__ __forceinline__ uint64_t ctl_of(uint64_t home, uint32_t d) {
+    return (home << 8) | ((uint64_t)d << 1);
+  }
+  // Whether the bucket of this control word owns hash h.
+  static __device__ __forceinline__ bool owns(uint64_t ctl, uint64_t h) {
+    return (h & mask(depth_of(ctl))) == home_of(ctl);
   }
 
-  // One attempt; on success `d` is the bucket's depth.  Lock users retry in
-  // a loop whose every iteration holds the whole critical section: a lane
-  // that gets the lock releases it in the same iteration, so lanes of one
+  // One attempt; on success `ctl` is the bucket's control word.  Lock users
+  // retry in a loop whose every iteration holds the whole critical section: a
+  // lane that gets the lock releases it in the same iteration, so lanes of one
   // wave waiting for the same bucket never keep its holder from running (a
   // spin-then-work loop would).
-  __device__ bool try_lock(bucket* b, uint32_t& d) {
-    const uint64_t old = gallatin::utils::atomic_or(&b->ctl, (uint64_t)1);
-    d = depth_of(old);
-    return (old & 1) == 0;
+  __device__ bool try_lock(bucket* b, uint64_t& ctl) {
+    ctl = gallatin::utils::atomic_or(&b->ctl, (uint64_t)1);
+    return (ctl & 1) == 0;
   }
 
-  __device__ void unlock(bucket* b, uint32_t d) {
+  __device__ void unlock(bucket* b, uint64_t ctl) {
     __builtin_amdgcn_s_waitcnt(0);  // the critical section's stores land first
-    gallatin::utils::atomic_store(&b->ctl, (uint64_t)d << 32);
+    gallatin::utils::atomic_store(&b->ctl, ctl);
   }
 
   // Split full bucket b (locked, depth d): keys with bit d set move to a new
@@ -312,15 +420,14 @@ struct extendible_hash_table {
       if (go) st(&nb->vals[s], v[s]);
       st(&nb->keys[s], go ? k[s] : (uint64_t)defaultKey);
     }
-    st(&nb->ctl, (uint64_t)(d + 1) << 32);
-    st(&nb->home, home);
+    st(&nb->ctl, ctl_of(home, d + 1));
     __builtin_amdgcn_s_waitcnt(0);  // the new bucket is whole before it is published
     st(reinterpret_cast<uint64_t*>(&directory[home]), reinterpret_cast<uint64_t>(nb));
     // level only grows: a cached value at or above d + 1 needs no update
     if (ld_cached(&level) < d + 1)
       gallatin::utils::atomic_max(&level, (uint64_t)(d + 1));
     __builtin_amdgcn_s_waitcnt(0);
-    st(&b->ctl, ((uint64_t)(d + 1) << 32) | 1);  // still locked
+    st(&b->ctl, ctl_of(old_home, d + 1) | 1);  // still locked
     __builtin_amdgcn_s_waitcnt(0);  // new depth visible before keys leave
 #pragma unroll
     for (int s = 0; s < items_per_bucket; ++s)
@@ -328,61 +435,99 @@ struct extendible_hash_table {
     return true;
   }
 
-  // extendible_ht.cuh:842-1115.  Insert or replace; false when the table
-  // cannot hold the key.
-  __device__ bool insert(Key key, Val val) {
-    if ((uint64_t)key == (uint64_t)defaultKey || (uint64_t)key == (uint64_t)tombstoneKey)
-      return false;
+  // Insert (or replace) the pair of every lane with `put`, remove the key of
+  // every other; true when stored or found.  The operations of a wave run
+  // together, whichever they are, so that the lanes can read buckets together
+  // (scan); a lane that is done stays in the loop for the others.
+  __device__ bool update(bool put, Key key, Val val) {
+    const bool valid = !put || ((uint64_t)key != (uint64_t)defaultKey &&
+                                (uint64_t)key != (uint64_t)tombstoneKey);
     const uint64_t h = hash(key);
-    int state = 0;  // 0 pending, 1 stored, 2 refused
-    for (uint32_t tries = 0; state == 0 && tries < kTries; ++tries) {
-      bucket* b = owner(h, tries > 0);
-      if (!b) {
-        state = 2;
-        break;
-      }
-      uint32_t d;
-      if (!try_lock(b, d)) {
-        __builtin_amdgcn_s_sleep(2);
-        continue;
+    int state = valid ? 0 : 3;  // 0 pending, 1 done, 2 refused or absent, 3 not a key
+    bucket* b = nullptr;
+    bool fresh = false;
+    uint32_t losses = 0;
+    for (uint32_t tries = 0; __ballot(state == 0) && tries < kTries; ++tries) {
+      uint64_t ctl = 0;
+      bool held = false;
+      if (state == 0) {
+        if (!b) {
+          b = owner(h, fresh);
+          fresh = true;
+        }
+        if (!b)
+          state = 2;
+        else
+          held = try_lock(b, ctl);
       }
       int match, free_slot;
-      const uint64_t home = scan(b, (uint64_t)key, match, free_slot);
-      if ((h & mask(d)) == home) {  // still the owner
+      uint64_t seen;
+      scan(held, b, (uint64_t)key, seen, match, free_slot);
+      if (held) {
+        if (!owns(ctl, h)) {
+          unlock(b, ctl);
+          b = nullptr;  // split since the look-up: look again
+          continue;
+        }
         if (match >= 0) {
-          st(&b->vals[match], (uint64_t)val);
+          if (put)
+            st(&b->vals[match], (uint64_t)val);
+          else
+            st(&b->keys[match], (uint64_t)defaultKey);
           state = 1;
+        } else if (!put) {
+          state = 2;
         } else if (free_slot >= 0) {
           st(&b->vals[free_slot], (uint64_t)val);
           __builtin_amdgcn_s_waitcnt(0);  // value before key
           st(&b->keys[free_slot], (uint64_t)key);
           state = 1;
-        } else if (d < max_bits && split(b, d, home)) {  // full: split, try again
-          d += 1;
+        } else if (depth_of(ctl) < max_bits && split(b, depth_of(ctl), home_of(ctl))) {
+          ctl = ctl_of(home_of(ctl), depth_of(ctl) + 1);  // full: split, try again
         } else {
           state = 2;
         }
+        unlock(b, ctl);
+        if (state == 0) b = nullptr;
+      } else if (state == 0) {
+        // Locked: the same bucket again a few times, then look up again, which
+        // also keeps the waiting lanes off the word that the holder has to
+        // unlock.  Trying the same bucket until its word shows a split took
+        // 20 ms where this takes 7 (200,000 keys into 16 first buckets);
+        // looking up every time, 1,000 keys in 600 buckets take 56 us, not 50.
+        if (++losses > kSameBucket || !owns(ctl, h)) b = nullptr;
+        __builtin_amdgcn_s_sleep(2);
       }
-      unlock(b, d);
     }
-    if (state != 1) gallatin::utils::atomic_add(&failed, (uint64_t)1);
+    if (put && (state == 0 || state == 2)) gallatin::utils::atomic_add(&failed, (uint64_t)1);
     return state == 1;
   }
 
-  // extendible_ht.cuh:1291-1375.  The depth, home and keys are loaded
+  // extendible_ht.cuh:842-1115.  Insert or replace; false when the table
+  // cannot hold the key.
+  __device__ bool insert(Key key, Val val) { return update(true, key, val); }
+
+  // Remove key; true if it was present.  (No counterpart in the reference.)
+  __device__ bool remove(Key key) { return update(false, key, Val{}); }
+
+  // extendible_ht.cuh:1291-1375.  The control word and the keys are loaded
   // together; a missing key is reported only if the depth is unchanged
   // when looked at again after the keys (a split raises the depth before
   // it clears moved keys), and a found key's value is taken only if the
   // key is still in its slot after the value was read.
   __device__ bool query(Key key, Val& val) {
     const uint64_t h = hash(key);
-    for (uint32_t tries = 0; tries < kTries; ++tries) {
-      bucket* b = owner(h, tries > 0);
-      if (!b) return false;
-      const uint32_t d0 = depth_of(ld(&b->ctl));
+    bool pending = true, found = false;
+    for (uint32_t tries = 0; __ballot(pending) && tries < kTries; ++tries) {
+      bucket* b = nullptr;
+      if (pending) {
+        b = owner(h, tries > 0);
+        pending = b != nullptr;
+      }
+      uint64_t ctl;
       int match, empty;
-      const uint64_t home = scan(b, (uint64_t)key, match, empty);
-      if ((h & mask(d0)) != home) continue;  // being split: look again
+      scan(pending, b, (uint64_t)key, ctl, match, empty);
+      if (!pending || !owns(ctl, h)) continue;  // being split: look again
       if (match >= 0) {
         const uint64_t v = ld(&b->vals[match]);
         __builtin_amdgcn_s_waitcnt(0);  // the value is read before the key is read again
@@ -391,39 +536,14 @@ struct extendible_hash_table {
         // first: the value belongs to the key only if the key is still there.
         if (ld(&b->keys[match]) == (uint64_t)key) {
           val = (Val)v;
-          return true;
+          found = true;
+          pending = false;
         }
-        continue;
+      } else if (depth_of(ld(&b->ctl)) == depth_of(ctl)) {
+        pending = false;
       }
-      if (depth_of(ld(&b->ctl)) == d0) return false;
     }
-    return false;
-  }
-
-  // Remove key; true if it was present.  (No counterpart in the reference.)
-  __device__ bool remove(Key key) {
-    const uint64_t h = hash(key);
-    int state = 0;  // 0 pending, 1 removed, 2 absent
-    for (uint32_t tries = 0; state == 0 && tries < kTries; ++tries) {
-      bucket* b = owner(h, tries > 0);
-      if (!b) break;
-      uint32_t d;
-      if (!try_lock(b, d)) {
-        __builtin_amdgcn_s_sleep(2);
-        continue;
-      }
-      int match, empty;
-      const uint64_t home = scan(b, (uint64_t)key, match, empty);
-      if ((h & mask(d)) == home) {
-        state = 2;
-        if (match >= 0) {
-          st(&b->keys[match], (uint64_t)defaultKey);
-          state = 1;
-        }
-      }
-      unlock(b, d);
-    }
-    return state == 1;
+    return found;
   }
 };
 

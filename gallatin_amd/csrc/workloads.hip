@@ -21,94 +21,7 @@ using namespace gallatin_capi;
 namespace {
 
 #include "lane_counts.hpp"
-
-// Payload fill and verify, spread over the whole wave: the buffers of the
-// participating lanes are cut into 16-byte chunks numbered buffer after
-// buffer (lane order), and lane r handles chunks r, r + 64, r + 128, ...
-// A chunk's owner is the last lane whose chunk prefix is <= the chunk index,
-// found by a 6-step binary search over the prefixes (one per lane, read with
-// ds_bpermute).  Needs all 64 lanes of the wave active; the chunk loops are
-// wave-uniform (every lane takes part in every ds_bpermute, a disabled source
-// lane would read as 0) and only the memory access itself is predicated.
-//
-// A buffer of w words (w = ceil(size / 8)) lives in a slice whose size is a
-// multiple of 16 bytes and at least 8 * w, so for odd w the slice extends at
-// least 8 bytes past the last word: every chunk is accessed as one aligned
-// 16-byte vector, and the verify ignores the upper half of a buffer's last
-// chunk when w is odd.  Accesses go through global-address-space pointers
-// (global_load / global_store), so stores never hold up the LDS waits of the
-// owner search, and the verify keeps kVerifyDepth loads per lane in flight.
-typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) u64x2 global_u64x2;
-
-constexpr int kVerifyDepth = 8;
-
-struct chunk_plan {
-  uint32_t prefix;    // chunks owned by lower lanes
-  uint32_t total;     // chunks of the whole wave
-  uint32_t full_end;  // chunks below this index of this lane's buffer are full
-  uint64_t adjusted;  // buffer address - 16 * prefix
-};
-
-__device__ inline chunk_plan plan_chunks(bool on, const void* p, uint64_t words) {
-  const uint32_t n = on ? (uint32_t)((words + 1) / 2) : 0u;
-  chunk_plan c;
-  wave::group_scan(n, ~0ULL, c.prefix, c.total);
-  c.full_end = c.prefix + (on ? (uint32_t)(words / 2) : 0u);
-  c.adjusted = (uint64_t)p - 16ULL * c.prefix;
-  return c;
-}
-
-__device__ __forceinline__ int chunk_owner(uint32_t prefix, uint32_t c) {
-  int l = 0;
-  for (int step = 32; step; step >>= 1) {
-    const uint32_t p = wave::fetch(prefix, l + step);
-    if (p <= c) l += step;
-  }
-  return l;
-}
-
-__device__ inline void wave_fill(bool on, uint64_t* p, uint64_t words, uint64_t pat) {
-  const chunk_plan cp = plan_chunks(on, p, words);
-  const uint32_t lane = wave::lane();
-  for (uint32_t base = 0; base < cp.total; base += 64) {
-    const uint32_t c = base + lane;
-    const bool in = c < cp.total;
-    const int l = chunk_owner(cp.prefix, in ? c : cp.total - 1);
-    const uint64_t a = wave::fetch(cp.adjusted, l) + 16ULL * c;
-    const uint64_t v = wave::fetch(pat, l);
-    if (in) *reinterpret_cast<global_u64x2*>(a) = u64x2{v, v};
-  }
-}
-
-// Returns this lane's share of the mismatching words.
-__device__ inline uint32_t wave_verify(bool on, const uint64_t* p, uint64_t words,
-                                       uint64_t pat) {
-  const chunk_plan cp = plan_chunks(on, p, words);
-  const uint32_t lane = wave::lane();
-  uint32_t bad = 0;
-  for (uint32_t base = 0; base < cp.total; base += 64 * kVerifyDepth) {
-    uint64_t a[kVerifyDepth], v[kVerifyDepth];
-    bool in[kVerifyDepth], full[kVerifyDepth];
-#pragma unroll
-    for (int k = 0; k < kVerifyDepth; ++k) {
-      const uint32_t c = base + 64u * k + lane;
-      in[k] = c < cp.total;
-      const int l = chunk_owner(cp.prefix, in[k] ? c : cp.total - 1);
-      a[k] = wave::fetch(cp.adjusted, l) + 16ULL * c;
-      v[k] = wave::fetch(pat, l);
-      full[k] = c < wave::fetch(cp.full_end, l);
-    }
-    u64x2 x[kVerifyDepth];
-#pragma unroll
-    for (int k = 0; k < kVerifyDepth; ++k)
-      if (in[k]) x[k] = *reinterpret_cast<const global_u64x2*>(a[k]);
-#pragma unroll
-    for (int k = 0; k < kVerifyDepth; ++k)
-      if (in[k]) bad += (x[k].x != v[k]) + (full[k] && x[k].y != v[k]);
-  }
-  return bad;
-}
+#include "payload.hpp"
 
 }  // namespace
 
@@ -184,6 +97,8 @@ __global__ void k_plain(gal_state* s, uint64_t n, uint64_t size, uint64_t* ctr) 
 // every later round whose coin is set, and freed after the last round.
 __global__ void k_churn(gal_state* s, uint64_t seed, uint64_t n, uint32_t rounds,
                         uint64_t* ctr) {
+  extern __shared__ chunk_map maps[];  // one per wave
+  chunk_map& m = maps[wave::readfirst(threadIdx.x >> 6)];
   const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool active = tid < n;
   uint64_t* live = nullptr;
@@ -194,7 +109,7 @@ __global__ void k_churn(gal_state* s, uint64_t seed, uint64_t n, uint32_t rounds
     const bool replace =
         active && (r == 0 || r == rounds || gal_churn_coin(seed, tid, r) != 0);
     const bool do_free = replace && live != nullptr;
-    c.bad += wave_verify(do_free, live, live_words, gal_churn_pattern(tid, live_round));
+    c.bad += wave_verify(m, do_free, live, live_words, gal_churn_pattern(tid, live_round));
     if (do_free) {
       detail::free_impl(s, live);
       c.pairs += 1;
@@ -216,7 +131,7 @@ __global__ void k_churn(gal_state* s, uint64_t seed, uint64_t n, uint32_t rounds
       live_round = r;
       c.bytes += (uint64_t)live_words * 8;
     }
-    wave_fill(filled, np, gal_fill_words(size), gal_churn_pattern(tid, r));
+    wave_fill(m, filled, np, gal_fill_words(size), gal_churn_pattern(tid, r));
   }
   add_counters(ctr, c);
 }
@@ -268,6 +183,8 @@ __global__ __launch_bounds__(kThreads) void k_churn_batched(gal_state* s, uint64
                                                             uint64_t n, uint32_t rounds,
                                                             uint64_t* ctr) {
   __shared__ batch::lds_state lds;
+  __shared__ chunk_map maps[kThreads / 64];
+  chunk_map& m = maps[wave::readfirst(threadIdx.x >> 6)];
   batch::batch_init(lds);
   lane_counts c;
   const uint64_t nchunks = (n + blockDim.x - 1) / blockDim.x;
@@ -281,7 +198,7 @@ __global__ __launch_bounds__(kThreads) void k_churn_batched(gal_state* s, uint64
       const bool replace =
           active && (r == 0 || r == rounds || gal_churn_coin(seed, tid, r) != 0);
       const bool do_free = replace && live != nullptr;
-      c.bad += wave_verify(do_free, live, live_words, gal_churn_pattern(tid, live_round));
+      c.bad += wave_verify(m, do_free, live, live_words, gal_churn_pattern(tid, live_round));
       void* old = do_free ? live : nullptr;
       if (do_free) {
         c.pairs += 1;
@@ -305,7 +222,7 @@ __global__ __launch_bounds__(kThreads) void k_churn_batched(gal_state* s, uint64
         live_round = r;
         c.bytes += (uint64_t)live_words * 8;
       }
-      wave_fill(filled, np, gal_fill_words(size), gal_churn_pattern(tid, r));
+      wave_fill(m, filled, np, gal_fill_words(size), gal_churn_pattern(tid, r));
     }
   }
   add_counters(ctr, c);
@@ -471,7 +388,8 @@ int gal_run_churn(gal_allocator* a, uint64_t seed, uint64_t n, uint32_t rounds,
   if (!a || !ctr) return fail(GAL_ERR_INVALID, "null argument");
   if (n == 0) return GAL_OK;
   if (threads == 0 || threads > 1024 || threads % 64) threads = 256;
-  k_churn<<<grid_for(n, threads), threads, 0, (hipStream_t)stream>>>(a->dev, seed, n, rounds, ctr);
+  const size_t lds = threads / 64 * sizeof(chunk_map);
+  k_churn<<<grid_for(n, threads), threads, lds, (hipStream_t)stream>>>(a->dev, seed, n, rounds, ctr);
   return launch_status("churn");
 }
 

@@ -353,7 +353,7 @@ class Gallatin:
     def malloc_bulk(self, sizes, block_threads=256):
         """sizes: int64 cuda tensor -> int64 cuda tensor of device pointers."""
         import torch
-        out = torch.zeros(sizes.numel(), dtype=torch.int64, device="cuda")
+        out = torch.empty(sizes.numel(), dtype=torch.int64, device="cuda")
         _check(lib().gal_malloc_bulk(self.handle, sizes.data_ptr(), sizes.numel(),
                                      out.data_ptr(), block_threads, _stream()))
         return out
@@ -518,6 +518,9 @@ def run_batches(alloc, stream, counters=None, threads=0, batched=True, workgroup
     return ctr
 
 
+# Results are torch.empty: every kernel writes all of its n results, and a fill
+# before it is a launch of its own (about 5 us, a tenth of a batch of 1,000
+# keys through the hash table).
 # ---- allocator-backed data structures (on the global allocator) ----
 class Vector:
     """fixed_vector<uint64_t, 64, 2^22> (fixed_vector.cuh:72-512)."""
@@ -555,22 +558,22 @@ class Table:
 
     def insert(self, keys, vals):
         import torch
-        ok = torch.zeros(keys.numel(), dtype=torch.uint8, device="cuda")
+        ok = torch.empty(keys.numel(), dtype=torch.uint8, device="cuda")
         _check(lib().gal_table_insert(self.handle, keys.data_ptr(), vals.data_ptr(),
                                       keys.numel(), ok.data_ptr(), _stream()))
         return ok
 
     def query(self, keys):
         import torch
-        vals = torch.zeros(keys.numel(), dtype=torch.int64, device="cuda")
-        found = torch.zeros(keys.numel(), dtype=torch.uint8, device="cuda")
+        vals = torch.empty(keys.numel(), dtype=torch.int64, device="cuda")
+        found = torch.empty(keys.numel(), dtype=torch.uint8, device="cuda")
         _check(lib().gal_table_query(self.handle, keys.data_ptr(), keys.numel(),
                                      vals.data_ptr(), found.data_ptr(), _stream()))
         return vals, found
 
     def remove(self, keys):
         import torch
-        ok = torch.zeros(keys.numel(), dtype=torch.uint8, device="cuda")
+        ok = torch.empty(keys.numel(), dtype=torch.uint8, device="cuda")
         _check(lib().gal_table_remove(self.handle, keys.data_ptr(), keys.numel(),
                                       ok.data_ptr(), _stream()))
         return ok
@@ -618,7 +621,7 @@ class ChainTable:
         self._check_arg(vals)
         if keys.numel() != vals.numel():
             raise GallatinError("keys and values differ in length")
-        ok = torch.zeros(keys.numel(), dtype=torch.uint8, device="cuda")
+        ok = torch.empty(keys.numel(), dtype=torch.uint8, device="cuda")
         _check(lib().gal_chain_insert(self.handle, keys.data_ptr(), vals.data_ptr(),
                                       keys.numel(), ok.data_ptr(), _stream()))
         return ok
@@ -626,15 +629,15 @@ class ChainTable:
     def query(self, keys):
         import torch
         self._check_arg(keys)
-        vals = torch.zeros(keys.numel(), dtype=self._dtype(), device="cuda")
-        found = torch.zeros(keys.numel(), dtype=torch.uint8, device="cuda")
+        vals = torch.empty(keys.numel(), dtype=self._dtype(), device="cuda")
+        found = torch.empty(keys.numel(), dtype=torch.uint8, device="cuda")
         _check(lib().gal_chain_query(self.handle, keys.data_ptr(), keys.numel(),
                                      vals.data_ptr(), found.data_ptr(), _stream()))
         return vals, found
 
     def lengths(self):
         import torch
-        out = torch.zeros(self.nblocks, dtype=torch.int32, device="cuda")
+        out = torch.empty(self.nblocks, dtype=torch.int32, device="cuda")
         _check(lib().gal_chain_lengths(self.handle, out.data_ptr(), _stream()))
         return out
 
@@ -667,15 +670,15 @@ class BlockQueue:
 
     def enqueue(self, items, serial=False):
         import torch
-        ok = torch.zeros(items.numel(), dtype=torch.uint8, device="cuda")
+        ok = torch.empty(items.numel(), dtype=torch.uint8, device="cuda")
         _check(lib().gal_bqueue_enqueue(self.handle, items.data_ptr(), items.numel(),
                                         ok.data_ptr(), int(serial), _stream()))
         return ok
 
     def dequeue(self, n, serial=False):
         import torch
-        out = torch.zeros(n, dtype=torch.int64, device="cuda")
-        ok = torch.zeros(n, dtype=torch.uint8, device="cuda")
+        out = torch.empty(n, dtype=torch.int64, device="cuda")
+        ok = torch.empty(n, dtype=torch.uint8, device="cuda")
         _check(lib().gal_bqueue_dequeue(self.handle, out.data_ptr(), ok.data_ptr(), n,
                                         int(serial), _stream()))
         return out, ok
@@ -706,15 +709,15 @@ class Queue:
 
     def enqueue(self, items, serial=False):
         import torch
-        ok = torch.zeros(items.numel(), dtype=torch.uint8, device="cuda")
+        ok = torch.empty(items.numel(), dtype=torch.uint8, device="cuda")
         _check(lib().gal_queue_enqueue(self.handle, items.data_ptr(), items.numel(),
                                        ok.data_ptr(), int(bool(serial)), _stream()))
         return ok
 
     def dequeue(self, n, serial=False):
         import torch
-        out = torch.zeros(n, dtype=torch.int64, device="cuda")
-        ok = torch.zeros(n, dtype=torch.uint8, device="cuda")
+        out = torch.empty(n, dtype=torch.int64, device="cuda")
+        ok = torch.empty(n, dtype=torch.uint8, device="cuda")
         _check(lib().gal_queue_dequeue(self.handle, out.data_ptr(), ok.data_ptr(), n,
                                        int(bool(serial)), _stream()))
         return out, ok
@@ -754,7 +757,7 @@ def global_allocator():
 
 def global_malloc_bulk(sizes, block_threads=256):
     import torch
-    out = torch.zeros(sizes.numel(), dtype=torch.int64, device="cuda")
+    out = torch.empty(sizes.numel(), dtype=torch.int64, device="cuda")
     _check(lib().gal_global_malloc_bulk(sizes.data_ptr(), sizes.numel(),
                                         out.data_ptr(), block_threads, _stream()))
     return out
@@ -813,7 +816,7 @@ def print_global_stats_combined():
 
 def _ptrs_out(n):
     import torch
-    return torch.zeros(n, dtype=torch.int64, device="cuda")
+    return torch.empty(n, dtype=torch.int64, device="cuda")
 
 
 def global_malloc_fused_bulk(sizes):
@@ -848,7 +851,7 @@ def global_malloc_poison_bulk(sizes):
 
 def global_check_poison_bulk(ptrs):
     import torch
-    ok = torch.zeros(ptrs.numel(), dtype=torch.uint8, device="cuda")
+    ok = torch.empty(ptrs.numel(), dtype=torch.uint8, device="cuda")
     _check(lib().gal_global_check_poison_bulk(ptrs.data_ptr(), ptrs.numel(), ok.data_ptr(),
                                               _stream()))
     return ok

@@ -436,8 +436,10 @@ int gal_serving_destroy(gal_serving *s);
  * where slot was filled by an earlier batch.  Each allocation holds its slot
  * number in its first 8 bytes, checked at free (counter [2]; an op with a
  * slot >= nslots or an unknown kind also counts there and is skipped).  One
- * persistent launch per batch, then one launch freeing whatever is left in
- * ptrs[0 .. nslots), so the table is empty again at the end.  batched: 0
+ * persistent launch per batch (with batched 0 or 1, consecutive batches of at
+ * most 1024 or `threads` ops share one, in order), then one launch freeing
+ * whatever is left in ptrs[0 .. nslots), so the table is empty again at the
+ * end.  batched: 0
  * plain per-thread malloc/free; 1 the workgroup-batched path (batched.hpp);
  * 2 mallocs through each workgroup's LDS slice cache (slice_cache.hpp) and
  * per-wave frees.  threads: 256, 512 or 1024 (0 = 1024; modes 1 and 2

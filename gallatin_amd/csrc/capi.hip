@@ -310,11 +310,13 @@ int gal_create(const gal_config* cfg, gal_allocator** out) {
     const uint32_t c = (p + P - 1) / P * P;
     h.slot_off[t] = total;
     h.slot_count[t] = c;
+    h.slot_part[t] = c / P;
     total += c;
     p /= 2;
     if (p < pmin) p = pmin;
   }
   h.slot_off[T] = total;
+  h.class_bits = T > 1 ? 32u - (uint32_t)__builtin_clz(T - 1) : 0u;
   h.total_slots = total;
   // trees: segment tree + one per class and partition, in one word arena
   uint64_t words = 0;

@@ -158,6 +158,21 @@ __device__ __forceinline__ uint64_t match(uint64_t cand, bool in, uint64_t key) 
   return mine;
 }
 
+// match for keys below 2^bits: a ballot per bit of the key instead of one per
+// distinct key (a churn wave holds nine size classes, four bits).
+__device__ __forceinline__ uint64_t match_bits(uint64_t cand, bool in, uint32_t key,
+                                               uint32_t bits) {
+  uint32_t lo = (uint32_t)cand, hi = (uint32_t)(cand >> 32);
+  for (uint32_t b = 0; b < bits; ++b) {
+    const bool one = (key >> b) & 1u;
+    const uint64_t m = __ballot(one);
+    const uint32_t flip = one ? 0u : ~0u;  // lanes whose bit differs drop out
+    lo &= (uint32_t)m ^ flip;
+    hi &= (uint32_t)(m >> 32) ^ flip;
+  }
+  return in ? ((uint64_t)hi << 32) | lo : 0;
+}
+
 // Sum of `v` over the lanes of `group` that lie below this lane (exclusive
 // prefix) and over the whole group, from bit-sliced ballots.  Exact for any
 // exec mask; `max_bits` bounds the values.  Replaces cg::exclusive_scan and

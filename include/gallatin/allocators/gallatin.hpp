@@ -71,7 +71,9 @@ __device__ __forceinline__ bool deterministic(const gal_state* s) {
 
 // Partition of the calling wave: its XCD (__smid() = xcc << 6 | se << 4 | cu).
 __device__ __forceinline__ uint32_t wave_part(const gal_state* s) {
-  return s->num_parts == 1 ? 0u : (__smid() >> 6) % s->num_parts;
+  if (s->num_parts == 1) return 0u;
+  const uint32_t x = __smid() >> 6;
+  return x < s->num_parts ? x : x % s->num_parts;  // a division is 20 instructions
 }
 
 __device__ __forceinline__ const gal_tree& class_tree(const gal_state* s, uint32_t t,
@@ -435,12 +437,12 @@ __device__ __noinline__ void free_segments(gal_state* s, uint64_t seg, uint64_t 
 // without a block (at most 30 steps).  Returns (slot << 32) | block; with no
 // block found, the start slot and its content (kNullBlock or kRefilling).
 __device__ inline uint64_t pinned_block(const gal_state* s, uint32_t t, uint32_t p) {
-  const uint32_t per = s->slot_count[t] / s->num_parts;
+  const uint32_t per = s->slot_part[t];
   const uint32_t base = p * per;
   uint32_t rel = 0;
   if (!deterministic(s)) {
     const uint32_t mix = ((__smid() & 63u) * 0x9E3779B1u) >> 26;  // 0..63
-    rel = mix % per;
+    rel = (mix * per) >> 6;  // the CUs spread evenly over the slots
   }
   const uint32_t* sl = s->slots + s->slot_off[t] + base;
   const int64_t original = rel;
@@ -449,7 +451,7 @@ __device__ inline uint64_t pinned_block(const gal_state* s, uint32_t t, uint32_t
   const uint32_t first = blk;
   int counter = 0;
   while (blk >= kRefilling && i != original - 1) {
-    i = (i + 1) % per;
+    i = i + 1 < per ? i + 1 : 0;
     blk = atomic_load(&sl[i]);
     if (++counter >= kSlotScanCutoff) break;
   }
@@ -754,7 +756,7 @@ __device__ __forceinline__ void malloc_slices(gal_state* s, bool want, uint32_t 
     const uint64_t pend = __ballot(pending);
     if (!pend) break;
     // coalesced groups by class (labeled_partition, gallatin.cuh:883-885)
-    const uint64_t grp = wave::match(pend, pending, t);
+    const uint64_t grp = wave::match_bits(pend, pending, t, s->class_bits);
     const int leader = pending ? wave::first(grp) : (int)lane;
     const bool is_leader = pending && leader == (int)lane;
     uint64_t sb = kNullBlock;

@@ -182,6 +182,8 @@ struct gal_state {
   uint32_t slot_off[kMaxTrees + 1];
   uint32_t slot_count[kMaxTrees];  // multiple of num_parts; partition p owns
                                    // slots [p, p+1) * count / num_parts
+  uint32_t slot_part[kMaxTrees];   // slot_count / num_parts
+  uint32_t class_bits;             // bits of a class number: classes < 2^class_bits
   gal_tree seg_tree;
   gal_tree sub_trees[kMaxTrees * kMaxParts];  // class t, partition p at t*parts+p
   // `table` of the reference's Gallatin (gallatin.cuh:306): the device

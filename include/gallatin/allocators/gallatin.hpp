@@ -709,6 +709,7 @@ __device__ __noinline__ uint32_t refill_slot(gal_state* s, uint32_t t, uint32_t 
   bool emptied;
   const uint32_t nb =
       request_new_blocks(s, t, p, det, s->lim_request, wave::is_first(), emptied);
+  release_to_xcd();  // see replace_block
   if (wave::is_first()) {
     atomic_exch(sp, nb);  // the block, or empty again
     if (nb != kNullBlock) add_stat(s, kStatRefills, 1);
@@ -737,6 +738,12 @@ __device__ __noinline__ void replace_block(gal_state* s, uint32_t t, uint32_t p,
   bool emptied;
   const uint32_t nb =
       request_new_blocks(s, t, p, det, s->lim_request, wave::is_first(), emptied);
+  // The block's counter is cleared before its id can be read from the slot.
+  // Waves that still add to the block's last incarnation can hold the
+  // clearing exchange back for tens of microseconds; a helper that found the
+  // id in the slot and the old, full count behind it would detach the block
+  // without retiring it, and its segment would never come back.
+  release_to_xcd();
   if (wave::is_first()) atomic_exch(sp, nb);
   // the waves waiting for the slot have their block; the set-up of the next
   // segment takes a lock and about 10 us

@@ -26,3 +26,21 @@ def test_churn_payload_around_the_sharing_threshold(gpu, n, partitions, batched)
     a.drain()
     H.check_fresh(a)
     a.free_on_device()
+
+
+def test_pinned_blocks_come_back_from_a_slow_pool(gpu):
+    """Waves of a launch that allocates and frees at once add to full blocks
+    while they are replaced; a pool in host memory holds them up longest.
+    Every block pinned meanwhile is accounted for afterwards."""
+    import torch
+    for k in range(12):
+        a = gpu.Gallatin(16 << 20, 16, 4096).generate_on_device_host(4 << 30, 42,
+                                                                    print_info=False)
+        try:
+            a.run_plain(1 << 18, 16)
+            a.run_churn(5 + k, 1 << 16, 4)
+            torch.cuda.synchronize()
+            a.drain()
+            H.check_fresh(a)
+        finally:
+            a.free_on_device()

@@ -31,11 +31,7 @@ using namespace gallatin_capi;
 
 namespace {
 
-__device__ inline uint64_t wave_total(uint64_t v) {
-  for (int off = 32; off >= 1; off >>= 1)
-    v += wave::fetch(v, (int)(wave::lane() ^ (uint32_t)off));
-  return v;
-}
+#include "lane_counts.hpp"
 
 struct op_counts {
   uint64_t pairs = 0, misses = 0, bad = 0, bytes = 0, mallocs = 0, skipped = 0;
@@ -46,30 +42,25 @@ struct op_counts {
   uint64_t malloc_ticks = 0, wait_ticks = 0, free_ticks = 0, start = wall_clock64();
 };
 
-// One atomic per counter per wave (every lane of the wave active).  The
-// wave's time split is added once per wave (lane 0's clock readings), with
-// its lifetime when `timed`.
+// The wave's time split is added once per wave (lane 0's clock readings),
+// with its lifetime when `timed`.
 __device__ inline void flush_counts(uint64_t* ctr, const op_counts& c, bool timed = false) {
-  const uint64_t v[5] = {wave_total(c.pairs), wave_total(c.misses), wave_total(c.bad),
-                         wave_total(c.bytes), wave_total(c.mallocs)};
-  const uint64_t sk = wave_total(c.skipped);
-  const uint64_t polls = wave_total(c.polls);
+  uint64_t v[GAL_CTR_COUNT] = {};
   const uint64_t life = wall_clock64() - c.start;
-  if (wave::lane() == 0) {
-#pragma unroll
-    for (int i = 0; i < 5; ++i)
-      if (v[i]) utils::atomic_add(&ctr[i], v[i]);
-    if (sk) utils::atomic_add(&ctr[GAL_CTR_FREES_SKIPPED], sk);
-    if (polls) utils::atomic_add(&ctr[GAL_CTR_WAIT_POLLS], polls);
-    if (timed) {
-      const uint64_t t[4] = {c.wait_ticks, life, c.malloc_ticks, c.free_ticks};
-      const int at[4] = {GAL_CTR_WAIT_TICKS, GAL_CTR_WAVE_TICKS, GAL_CTR_MALLOC_TICKS,
-                         GAL_CTR_FREE_TICKS};
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (t[i]) utils::atomic_add(&ctr[at[i]], t[i]);
-    }
+  v[GAL_CTR_PAIRS] = wave_sum(c.pairs);
+  v[GAL_CTR_MISSES] = wave_sum(c.misses);
+  v[GAL_CTR_BAD] = wave_sum(c.bad);
+  v[GAL_CTR_BYTES] = wave_sum(c.bytes);
+  v[GAL_CTR_MALLOCS] = wave_sum(c.mallocs);
+  v[GAL_CTR_FREES_SKIPPED] = wave_sum(c.skipped);
+  v[GAL_CTR_WAIT_POLLS] = wave_sum(c.polls);
+  if (timed) {
+    v[GAL_CTR_WAIT_TICKS] = c.wait_ticks;
+    v[GAL_CTR_WAVE_TICKS] = life;
+    v[GAL_CTR_MALLOC_TICKS] = c.malloc_ticks;
+    v[GAL_CTR_FREE_TICKS] = c.free_ticks;
   }
+  add_wave_totals(ctr, v);
 }
 
 // Pointer table protocol.  An entry is 0 until its malloc has run, then

@@ -775,14 +775,11 @@ struct gal_serving {
 
 namespace {
 
-// Adds the number of active lanes with `pred` set to *c with one atomic per
-// wave.  Every active lane must call it.  Per-lane atomics on one shared
-// counter serialise at one memory channel (about 88 M/s on MI355X), which
-// would dominate a kernel of a million short operations.
-__device__ __forceinline__ void count_wave(uint64_t* c, bool pred) {
-  const uint64_t m = __ballot(pred);
-  if (m && gallatin::wave::is_first())
-    gallatin::utils::atomic_add(c, (uint64_t)gallatin::wave::count(m));
+#include "lane_counts.hpp"
+
+// Lanes of the wave with `pred`.
+__device__ __forceinline__ uint64_t count_wave(bool pred) {
+  return gallatin::wave::count(__ballot(pred));
 }
 
 __device__ __forceinline__ uint64_t mix3(uint64_t a, uint64_t b, uint64_t c) {
@@ -936,15 +933,10 @@ __global__ __launch_bounds__(256) void k_serve_sessions(serving_session* ss, uin
     }
     if (live) words += end - at;
   }
-  const uint64_t vals[6] = {ended, words, refused, chunks, chunk_fail, freed};
-  const int idx[6] = {kSrvEnded, kSrvWords, kSrvWordsRefused, kSrvChunks, kSrvChunkFailed,
-                      kSrvChunksFreed};
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    uint64_t t = vals[i];
-    for (int off = 32; off >= 1; off >>= 1) t += gallatin::wave::fetch(t, (int)(lane ^ (uint32_t)off));
-    if (lane == 0 && t) gallatin::utils::atomic_add(&ctr[idx[i]], t);
-  }
+  // kSrvEnded and the five counters after it
+  const uint64_t totals[6] = {wave_sum(ended),  wave_sum(words),      wave_sum(refused),
+                              wave_sum(chunks), wave_sum(chunk_fail), wave_sum(freed)};
+  add_wave_totals(ctr + kSrvEnded, totals);
 }
 
 // Free memory of the global allocator for the admission gate (one
@@ -990,13 +982,12 @@ __global__ void k_serve_admit(serving_session* ss, uint32_t* free_slots, int32_t
                               uint32_t arrivals, uint64_t reserve, uint32_t gate,
                               const uint64_t* free_segments, uint32_t step, uint64_t* ctr) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= arrivals) return;
   // One pop of the free-slot stack per wave: the wave takes as many slots
   // as it has arrivals, and the lanes past what the stack held give theirs
   // back.
   const uint64_t free_now =
       free_segments[0] + (gate ? free_segments[1] / global_gallatin->blocks_per_segment : 0);
-  const bool room = free_now > reserve;
+  const bool room = i < arrivals && free_now > reserve;
   const uint64_t want = __ballot(room);
   const uint32_t rank = gallatin::wave::count(want & gallatin::wave::lanes_below());
   int32_t top0 = 0;
@@ -1016,22 +1007,23 @@ __global__ void k_serve_admit(serving_session* ss, uint32_t* free_slots, int32_t
     se.vec.init();
     se.alive = 1;
   }
-  count_wave(&ctr[kSrvAdmitted], admitted);
-  count_wave(&ctr[kSrvRefused], !admitted);
+  const uint64_t totals[2] = {count_wave(admitted), count_wave(i < arrivals && !admitted)};
+  add_wave_totals(ctr + kSrvAdmitted, totals);
 }
 
 __global__ void k_serve_table(table_large* t, uint64_t seed, uint32_t step, uint32_t n,
                               uint64_t* ctr) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const bool in = i < n;
   const uint64_t r = mix3(seed ^ 0x5eedULL, step, i);
   const uint64_t key = (r & ((1ULL << 28) - 1)) + 1;
   const bool ins = (r >> 40) % 10 < 7;
-  const bool ok = t->update(ins, key, r);
-  count_wave(&ctr[kSrvHtInserted], ins && ok);
-  count_wave(&ctr[kSrvHtFailed], ins && !ok);
-  count_wave(&ctr[kSrvHtRemoved], !ins && ok);
-  count_wave(&ctr[kSrvHtAbsent], !ins && !ok);
+  bool ok = false;
+  if (in) ok = t->update(ins, key, r);
+  // kSrvHtInserted and the three counters after it
+  const uint64_t totals[4] = {count_wave(in && ins && ok), count_wave(in && !ins && ok),
+                              count_wave(in && !ins && !ok), count_wave(in && ins && !ok)};
+  add_wave_totals(ctr + kSrvHtInserted, totals);
 }
 
 // One wave per live session (grid-stride): every word read back.  out[0]

@@ -830,24 +830,32 @@ __device__ __forceinline__ void write_words(uint64_t* w, uint64_t cs, uint64_t a
   if ((stop - at) & 1 && sl == 0) w[stop - 1 - cs] = tag | (stop - 1);
 }
 
-// Session pass: each wave takes 64 session slots at a time.
+// Session pass: each wave takes `per` session slots at a time (8 to 64).
+// The step is bound by a wave's serial work: a session's chunk requests are
+// a chain of atomics (1.1 us each), ending sessions are freed one after
+// another and four are written at a time, so fewer slots per wave end it
+// sooner until the waves no longer run all at once.  Step time with 64, 16,
+// 8 and 4 slots per wave: 147, 88, 75, 66 us (4096 sessions), 168, 113, 101,
+// 99 us (16384), 237, 244, 203, 210 us (65536), 385, 357, 344, 371 us
+// (131072), 579, 554, 595, 583 us (262144).
 __global__ __launch_bounds__(256) void k_serve_sessions(serving_session* ss, uint32_t n,
                                                         uint32_t* free_slots, int32_t* top,
                                                         uint32_t* queue, const uint32_t* tokens,
                                                         uint64_t seed, uint32_t step,
-                                                        uint32_t end_q32, uint64_t* ctr) {
+                                                        uint32_t end_q32, uint32_t per,
+                                                        uint64_t* ctr) {
   gal_state* g = global_gallatin;
   const uint32_t lane = gallatin::wave::lane();
   uint64_t ended = 0, words = 0, refused = 0, chunks = 0, chunk_fail = 0, freed = 0;
-  // waves take 64 slots at a time, grid-stride (the launch has about one
-  // wave per 64 slots, so a shared queue counter would only add atomics on
+  // waves take `per` slots at a time, grid-stride (the launch has one or two
+  // of these per wave, so a shared queue counter would only add atomics on
   // one address)
   const uint32_t wave_id = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
   (void)queue;
-  for (uint64_t base = (uint64_t)wave_id * 64; base < n; base += (uint64_t)nwaves * 64) {
+  for (uint64_t base = (uint64_t)wave_id * per; base < n; base += (uint64_t)nwaves * per) {
     const uint32_t slot = (uint32_t)base + lane;
-    bool alive = slot < n && ss[slot].alive;
+    bool alive = lane < per && slot < n && ss[slot].alive;
     const uint64_t id = alive ? ss[slot].id : 0;
     const uint64_t r = mix3(seed, id, step);
     const bool ends = alive && (uint32_t)r < end_q32;
@@ -1142,12 +1150,16 @@ int gal_serving_step(gal_serving* sv, uint32_t step, uint32_t arrivals, uint64_t
   if (ht_ops && (e = hipEventRecord(sv->fork, st)) != hipSuccess)
     return hip_fail(e, "serving fork");
   k_serve_reset<<<1, 64, 0, st>>>(sv->queue, sv->free_segments);
-  const uint32_t waves = (sv->max_sessions + 63) / 64;
+  // Slots per wave: 8, and more only past two waves for each that 8
+  // workgroups per CU hold (131072 slots on 256 CUs).
+  uint32_t per = 8;
+  while (per < 64 && ((uint64_t)sv->max_sessions + per - 1) / per > (uint64_t)cus * 64) per *= 2;
+  const uint32_t waves = (uint32_t)(((uint64_t)sv->max_sessions + per - 1) / per);
   uint32_t groups = (uint32_t)cus * 8;
   if (groups * 4 > waves) groups = (waves + 3) / 4;
   k_serve_sessions<<<groups, 256, 0, st>>>(sv->sessions, sv->max_sessions, sv->free_slots,
                                            sv->free_top, sv->queue, sv->tokens, sv->seed, step,
-                                           end_q32, counters_dev);
+                                           end_q32, per, counters_dev);
   if (ht_ops) {
     if ((e = hipStreamWaitEvent(sv->side, sv->fork, 0)) != hipSuccess)
       return hip_fail(e, "serving fork");

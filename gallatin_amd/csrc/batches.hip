@@ -71,6 +71,15 @@ __device__ inline void flush_counts(uint64_t* ctr, const op_counts& c, bool time
 // at the device, not held in a non-coherent cache), the tag store is
 // acknowledged before the entry is published, and the free reads the tag
 // only after it has seen the entry.
+//
+// A batch may free a slot and, later in the batch, fill it again.  The malloc
+// then finds the entry still in the table when its op is decoded, and
+// publishes once the free has taken it (bounded wait): published over it, the
+// pointer would be lost and the new one freed in its place; published before
+// the free's 0 lands, it would be wiped out.  The free comes first in op
+// order, so its workgroup serves it in an earlier round, or in the same one
+// before it waits for anything; all workgroups of a launch run at once
+// (batch_grid), so every such free is reached.
 constexpr uint64_t kMallocFailed = 1;
 
 // Decode op i without waiting: a malloc (want, size) or a free (is_free)
@@ -114,10 +123,9 @@ __device__ inline void* take_entry(uint64_t* ptrs, uint32_t slot, uint64_t v, op
 
 // The pointer a free op releases: taken out of the table (bounded wait
 // for its malloc to publish it), tag checked; nullptr when the malloc
-// failed or the wait ran out.
-__device__ inline void* wait_free(uint64_t* ptrs, uint32_t slot, op_counts& c,
+// failed or the wait ran out.  `v` is the entry as read last.
+__device__ inline void* wait_free(uint64_t* ptrs, uint32_t slot, uint64_t v, op_counts& c,
                                   uint32_t spin_cap, uint64_t* ctr) {
-  uint64_t v = utils::atomic_load(&ptrs[slot]);
   for (uint32_t spins = 0; v == 0; ++spins) {  // its malloc has not run yet
     if (spins >= spin_cap) {
       utils::atomic_add(&ctr[GAL_CTR_TIMEOUTS], (uint64_t)1);
@@ -130,15 +138,29 @@ __device__ inline void* wait_free(uint64_t* ptrs, uint32_t slot, op_counts& c,
   return take_entry(ptrs, slot, v, c);
 }
 
+// Bounded wait for the free that takes the entry found in the slot of a
+// malloc.
+__device__ __noinline__ void wait_taken(uint64_t* ptrs, uint32_t slot, uint32_t spin_cap,
+                                        uint64_t* ctr) {
+  for (uint32_t spins = 0; utils::atomic_load(&ptrs[slot]) != 0; ++spins) {
+    if (spins >= spin_cap) {
+      utils::atomic_add(&ctr[GAL_CTR_TIMEOUTS], (uint64_t)1);
+      return;
+    }
+    __builtin_amdgcn_s_sleep(4);
+  }
+}
+
 // Decode op i: the pointer to free (taken out of the table, tag checked) or
-// the size to allocate.
+// the size to allocate, with what the slot of a malloc holds.
 __device__ inline void take_op(const gal_batch_op* ops, uint64_t i, bool active,
                                uint64_t* ptrs, uint64_t nslots, op_counts& c, void*& old,
-                               bool& want, uint64_t& size, uint32_t& slot,
+                               bool& want, uint64_t& size, uint32_t& slot, uint64_t& held,
                                uint32_t spin_cap, uint64_t* ctr) {
   bool is_free = false;
   decode_op(ops, i, active, nslots, c, want, size, slot, is_free);
-  old = is_free ? wait_free(ptrs, slot, c, spin_cap, ctr) : nullptr;
+  held = want || is_free ? utils::atomic_load(&ptrs[slot]) : 0;
+  old = is_free ? wait_free(ptrs, slot, held, c, spin_cap, ctr) : nullptr;
 }
 
 __device__ inline void give_op(void* np, bool want, uint32_t slot, uint64_t* ptrs,
@@ -154,6 +176,15 @@ __device__ inline void give_op(void* np, bool want, uint32_t slot, uint64_t* ptr
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   if (want)
     utils::atomic_store(&ptrs[slot], np ? reinterpret_cast<uint64_t>(np) : kMallocFailed);
+}
+
+// give_op for a batch that may free and fill a slot: `held` is the entry of
+// a malloc's slot as take_op found it.
+__device__ inline void refill_op(void* np, bool want, uint32_t slot, uint64_t held,
+                                 uint64_t* ptrs, op_counts& c, uint32_t spin_cap,
+                                 uint64_t* ctr) {
+  if (want && held != 0) wait_taken(ptrs, slot, spin_cap, ctr);
+  give_op(np, want, slot, ptrs, c);
 }
 
 // One batch through the workgroup-batched path: a persistent grid walks
@@ -173,9 +204,10 @@ __global__ __launch_bounds__(kThreads) void k_batch_batched(gal_state* s, const 
     bool want;
     uint64_t size;
     uint32_t slot;
-    take_op(ops, i, i < n, ptrs, nslots, c, old, want, size, slot, spin_cap, ctr);
+    uint64_t held;
+    take_op(ops, i, i < n, ptrs, nslots, c, old, want, size, slot, held, spin_cap, ctr);
     void* np = batch::batch_step(s, old, want, size, lds);
-    give_op(np, want, slot, ptrs, c);
+    refill_op(np, want, slot, held, ptrs, c, spin_cap, ctr);
   }
   flush_counts(ctr, c);
 }
@@ -197,10 +229,11 @@ __global__ __launch_bounds__(kThreads) void k_batch_cached(gal_state* s, const g
     bool want;
     uint64_t size;
     uint32_t slot;
-    take_op(ops, i, i < n, ptrs, nslots, c, old, want, size, slot, spin_cap, ctr);
+    uint64_t held;
+    take_op(ops, i, i < n, ptrs, nslots, c, old, want, size, slot, held, spin_cap, ctr);
     if (old) detail::free_impl(s, old);
     void* np = cache::cache_malloc(s, lds, want, size);
-    give_op(np, want, slot, ptrs, c);
+    refill_op(np, want, slot, held, ptrs, c, spin_cap, ctr);
   }
   cache::cache_flush(s, lds);
   flush_counts(ctr, c);
@@ -219,11 +252,12 @@ __global__ __launch_bounds__(256) void k_batch_plain(gal_state* s, const gal_bat
     bool want;
     uint64_t size;
     uint32_t slot;
-    take_op(ops, i, i < n, ptrs, nslots, c, old, want, size, slot, spin_cap, ctr);
+    uint64_t held;
+    take_op(ops, i, i < n, ptrs, nslots, c, old, want, size, slot, held, spin_cap, ctr);
     if (old) detail::free_impl(s, old);
     void* np = nullptr;
     if (want) np = detail::malloc_impl(s, size);
-    give_op(np, want, slot, ptrs, c);
+    refill_op(np, want, slot, held, ptrs, c, spin_cap, ctr);
   }
   flush_counts(ctr, c);
 }
@@ -304,7 +338,7 @@ __global__ __launch_bounds__(kThreads) void k_run_plain(gal_state* s, const gal_
 #pragma unroll
       for (uint32_t k = 0; k < 2; ++k) {
         if (unseen[k])
-          old[k] = wait_free(ptrs, f_slot[k * kHalf + threadIdx.x - kHalf], c, spin_cap, ctr);
+          old[k] = wait_free(ptrs, f_slot[k * kHalf + threadIdx.x - kHalf], 0, c, spin_cap, ctr);
         if (old[k]) detail::free_impl(s, old[k]);
       }
     } else {
@@ -364,7 +398,8 @@ __global__ __launch_bounds__(kThreads) void k_run_batched(gal_state* s, const ga
     const uint64_t size = op.arg;
     at += run.ops[b];
     if (b + 1 < run.nbatches && threadIdx.x < run.ops[b + 1]) op = ops[at + threadIdx.x];
-    void* old = is_free ? wait_free(ptrs, slot, c, spin_cap, ctr) : nullptr;
+    void* old = nullptr;
+    if (is_free) old = wait_free(ptrs, slot, utils::atomic_load(&ptrs[slot]), c, spin_cap, ctr);
     void* np = batch::batch_step(s, old, want, size, lds);
     if (want) {
       c.mallocs += 1;
@@ -571,7 +606,8 @@ __global__ __launch_bounds__(kThreads) void k_stream(gal_state* s, const gal_bat
         slot = op.slot;
       }
       const uint64_t t1 = timed ? wall_clock64() : 0;
-      void* old = is_free ? wait_free(ptrs, slot, c, spin_cap, ctr) : nullptr;
+      void* old = nullptr;
+      if (is_free) old = wait_free(ptrs, slot, utils::atomic_load(&ptrs[slot]), c, spin_cap, ctr);
       const uint64_t t2 = timed ? wall_clock64() : 0;
       if (old) detail::free_impl(s, old);
       if (timed) {
@@ -657,24 +693,33 @@ unsigned fill_grid(K kernel, int threads, uint32_t workgroups) {
   return (unsigned)(cus * per_cu);
 }
 
+// Workgroups of one batch's launch: as many as its chunks, at most
+// `workgroups` where the caller gave a number, and never more than the device
+// holds at once (a malloc may wait for a free that another workgroup of the
+// launch serves).
+template <typename K>
+unsigned batch_grid(K kernel, int threads, uint64_t chunks, uint32_t workgroups) {
+  unsigned g = fill_grid(kernel, threads, 0);
+  if (workgroups && g > workgroups) g = workgroups;
+  return g > chunks ? (unsigned)chunks : g;
+}
+
 constexpr uint32_t kStreamSpinCap = 1u << 22;  // polls of a free waiting for its entry
 constexpr int kRunOps = 1024;  // largest batch of a run of per-thread batches
 
 template <int kThreads>
 void launch_batched(gal_state* s, const gal_batch_op* ops, uint64_t n, uint64_t* ptrs,
                     uint64_t nslots, uint64_t* ctr, uint32_t workgroups, hipStream_t st) {
-  unsigned g = fill_grid(k_batch_batched<kThreads>, kThreads, workgroups);
-  const uint64_t chunks = (n + kThreads - 1) / kThreads;
-  if (g > chunks) g = (unsigned)chunks;
+  const unsigned g = batch_grid(k_batch_batched<kThreads>, kThreads, (n + kThreads - 1) / kThreads,
+                                workgroups);
   k_batch_batched<kThreads><<<g, kThreads, 0, st>>>(s, ops, n, ptrs, nslots, ctr, kStreamSpinCap);
 }
 
 template <int kThreads>
 void launch_cached(gal_state* s, const gal_batch_op* ops, uint64_t n, uint64_t* ptrs,
                    uint64_t nslots, uint64_t* ctr, uint32_t workgroups, hipStream_t st) {
-  unsigned g = fill_grid(k_batch_cached<kThreads>, kThreads, workgroups);
-  const uint64_t chunks = (n + kThreads - 1) / kThreads;
-  if (g > chunks) g = (unsigned)chunks;
+  const unsigned g = batch_grid(k_batch_cached<kThreads>, kThreads, (n + kThreads - 1) / kThreads,
+                                workgroups);
   k_batch_cached<kThreads><<<g, kThreads, 0, st>>>(s, ops, n, ptrs, nslots, ctr, kStreamSpinCap);
 }
 
@@ -788,9 +833,7 @@ static int enqueue_stream(gal_allocator* a, const gal_batch_op* ops, const uint6
       continue;
     }
     if (batched == 0) {
-      unsigned g = fill_grid(k_batch_plain, 256, workgroups);
-      const uint64_t need = (n + 255) / 256;
-      if (g > need) g = (unsigned)need;
+      const unsigned g = batch_grid(k_batch_plain, 256, (n + 255) / 256, workgroups);
       k_batch_plain<<<g, 256, 0, st>>>(s, o, n, ptrs, nslots, ctr, kStreamSpinCap);
     } else if (batched == 1 && threads == 256) {
       launch_batched<256>(s, o, n, ptrs, nslots, ctr, workgroups, st);

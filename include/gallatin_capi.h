@@ -435,7 +435,10 @@ int gal_serving_destroy(gal_serving *s);
  * malloc(arg) into ptrs[slot]; kind 1: free(ptrs[slot]) (nullptr skipped),
  * where slot was filled by an earlier batch.  Each allocation holds its slot
  * number in its first 8 bytes, checked at free (counter [2]; an op with a
- * slot >= nslots or an unknown kind also counts there and is skipped).  One
+ * slot >= nslots or an unknown kind also counts there and is skipped).  A
+ * batch may free a slot and fill it again in a later op.  A free whose entry
+ * was never filled, and a malloc into an entry that nothing frees, wait for a
+ * bounded time and count in counter [5].  One
  * persistent launch per batch (with batched 0 or 1, consecutive batches of at
  * most 1024 or `threads` ops share one, in order), then one launch freeing
  * whatever is left in ptrs[0 .. nslots), so the table is empty again at the
@@ -458,8 +461,8 @@ int gal_run_batches(gal_allocator *a, const gal_batch_op *ops_dev,
 
 /* Validity of a stream on the host (ops in host memory).  Every op has
  * kind 0 or 1 and a slot below nslots; a slot is filled again only after
- * its pointer was freed, and a free names a slot whose malloc ran in an
- * earlier batch.  persistent != 0 adds the requirement of the plan below:
+ * its pointer was freed (by an earlier op, of the same batch too), and a free
+ * names a slot whose malloc ran in an earlier batch.  persistent != 0 adds the requirement of the plan below:
  * each slot is filled at most once in the stream.  GAL_ERR_INVALID names
  * the first op that breaks a rule (gal_last_error).  No reference
  * counterpart. */

@@ -333,7 +333,10 @@ __global__ __launch_bounds__(kThreads) void k_run_plain(gal_state* s, const gal_
         unseen[k] = v == 0;
         if (v) old[k] = take_entry(ptrs, f_slot[i], v, c);
       }
-      __builtin_amdgcn_s_waitcnt(0);  // the entries found are cleared
+      // the entries found are cleared before the mallocs are told
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_s_waitcnt(0);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
       if (wave::lane() == 0) atomicAdd(&taken[q], 1u);
 #pragma unroll
       for (uint32_t k = 0; k < 2; ++k) {

@@ -262,31 +262,32 @@ __global__ __launch_bounds__(256) void k_batch_plain(gal_state* s, const gal_bat
   flush_counts(ctr, c);
 }
 
-// A run of consecutive batches of at most kThreads ops each, served in order
-// by one workgroup, with a barrier between two batches where batches that
-// run alone have a launch boundary.  What bounds a small batch is its chain
-// of dependent accesses: entry, tag, free counter, pinned slot, claim,
-// publish, about 1 us each, and a launch adds as much again (100 batches of 1
-// to 4,096 ops, median 5: 1,130 us one by one, 830 us in runs).  The ops of
-// the next batch are read before the barrier, and tag and entry are stored
-// side by side: nothing reads either before the barrier, which waits for both.
+// A run of consecutive small batches, served in order by one workgroup, with
+// a barrier between two batches where batches that run alone have a launch
+// boundary.  What bounds a small batch is its chain of dependent accesses:
+// entry, tag, free counter, pinned slot, claim, publish, about 1 us each, and
+// a launch adds as much again (64 batches of 5 ops: 8.8 us each one by one,
+// 4.5 in a run).  The ops of the next batch are read before the barrier, and
+// tag and entry are stored side by side: nothing reads either before the
+// barrier, which waits for both.
 constexpr uint32_t kRunBatches = 128;
 struct batch_run {
   uint32_t nbatches;
   uint16_t ops[kRunBatches];  // ops of each batch
 };
 
-// Per thread: the frees of a batch run on the upper half of the waves and its
-// mallocs on the lower half, beside each other (one after the other a batch
-// took 7.4 us, now 6.5).  A malloc that finds no memory tries again after the
-// batch's frees, and publishes only after the batch's frees have taken the
-// entries they found, as when a wave freed before it allocated.
+// Per thread: the first waves serve a batch's mallocs and the ones after them
+// its frees, one request per thread, beside each other (one after the other a
+// batch took 7.4 us, beside each other 6.5).  A malloc that finds no memory
+// tries again after the batch's frees, and publishes only after the batch's
+// frees have taken the entries they found, as when a wave freed before it
+// allocated.  Mallocs and frees that fill a wave each in part need one wave
+// more than the batch has, so a batch is at most kThreads - 64 ops.
 template <int kThreads>
 __global__ __launch_bounds__(kThreads) void k_run_plain(gal_state* s, const gal_batch_op* ops,
                                                         batch_run run, uint64_t* ptrs,
                                                         uint64_t nslots, uint64_t* ctr,
                                                         uint32_t spin_cap) {
-  constexpr uint32_t kHalf = kThreads / 2;
   __shared__ uint64_t m_size[kThreads];
   __shared__ uint32_t m_slot[kThreads], f_slot[kThreads];
   __shared__ uint32_t nm[2], nf[2], taken[2], missed[2];  // by batch parity
@@ -317,59 +318,48 @@ __global__ __launch_bounds__(kThreads) void k_run_plain(gal_state* s, const gal_
     if (b + 1 < run.nbatches && threadIdx.x < run.ops[b + 1]) op = ops[at + threadIdx.x];
     __syncthreads();
     const uint32_t mallocs = nm[q], frees = nf[q];
+    const uint32_t mwaves = (mallocs + 63) / 64, fwaves = (frees + 63) / 64;
+    const uint32_t w = wave::readfirst(threadIdx.x >> 6);
     // the last readers of the other parity's words have come here
     if (threadIdx.x == 0) nm[q ^ 1] = nf[q ^ 1] = taken[q ^ 1] = missed[q ^ 1] = 0;
-    uint32_t none = 0;  // bit k: this thread's k-th malloc found no memory
-    if (threadIdx.x >= kHalf) {
-      // at most two frees per thread; those whose entry is not published yet
-      // (not so in a valid stream) wait for it after the others are taken
-      void* old[2] = {nullptr, nullptr};
-      bool unseen[2] = {false, false};
-#pragma unroll
-      for (uint32_t k = 0; k < 2; ++k) {
-        const uint32_t i = k * kHalf + threadIdx.x - kHalf;
-        if (i >= frees) continue;
+    bool none = false;  // this thread's malloc found no memory
+    if (w < mwaves) {
+      const bool mine = threadIdx.x < mallocs;
+      void* np = mine ? detail::malloc_impl(s, m_size[threadIdx.x]) : nullptr;
+      if (np) utils::atomic_store(static_cast<uint64_t*>(np), (uint64_t)m_slot[threadIdx.x]);
+      if (mine) c.mallocs += 1;
+      none = mine && !np;
+      while (__hip_atomic_load(&taken[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <
+             fwaves)
+        __builtin_amdgcn_s_sleep(1);
+      if (np) utils::atomic_store(&ptrs[m_slot[threadIdx.x]], reinterpret_cast<uint64_t>(np));
+      if (none) missed[q] = 1;
+    } else if (w < mwaves + fwaves) {
+      const uint32_t i = threadIdx.x - 64 * mwaves;
+      void* old = nullptr;
+      bool unseen = false;  // not published yet (not so in a valid stream)
+      if (i < frees) {
         const uint64_t v = utils::atomic_load(&ptrs[f_slot[i]]);
-        unseen[k] = v == 0;
-        if (v) old[k] = take_entry(ptrs, f_slot[i], v, c);
+        unseen = v == 0;
+        if (v) old = take_entry(ptrs, f_slot[i], v, c);
       }
-      // the entries found are cleared before the mallocs are told
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      __builtin_amdgcn_s_waitcnt(0);
+      __builtin_amdgcn_s_waitcnt(0);  // the entries found are cleared
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       if (wave::lane() == 0) atomicAdd(&taken[q], 1u);
-#pragma unroll
-      for (uint32_t k = 0; k < 2; ++k) {
-        if (unseen[k])
-          old[k] = wait_free(ptrs, f_slot[k * kHalf + threadIdx.x - kHalf], 0, c, spin_cap, ctr);
-        if (old[k]) detail::free_impl(s, old[k]);
-      }
-    } else {
-      for (uint32_t k = 0; k * kHalf < mallocs; ++k) {
-        const uint32_t i = k * kHalf + threadIdx.x;
-        const bool mine = i < mallocs;
-        void* np = mine ? detail::malloc_impl(s, m_size[i]) : nullptr;
-        if (np) utils::atomic_store(static_cast<uint64_t*>(np), (uint64_t)m_slot[i]);
-        if (mine) c.mallocs += 1;
-        if (mine && !np) none |= 1u << k;
-        while (__hip_atomic_load(&taken[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <
-               kHalf / 64)
-          __builtin_amdgcn_s_sleep(1);
-        if (np) utils::atomic_store(&ptrs[m_slot[i]], reinterpret_cast<uint64_t>(np));
-      }
-      if (none) missed[q] = 1;
+      // the others after those are taken
+      if (unseen) old = wait_free(ptrs, f_slot[i], 0, c, spin_cap, ctr);
+      if (old) detail::free_impl(s, old);
     }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);  // tags, entries and frees have landed
     __syncthreads();
     if (missed[q]) {
-      for (uint32_t k = 0; none >> k; ++k) {
-        if (!((none >> k) & 1)) continue;
-        const uint32_t i = k * kHalf + threadIdx.x;
-        void* np = detail::malloc_impl(s, m_size[i]);
+      if (none) {
+        void* np = detail::malloc_impl(s, m_size[threadIdx.x]);
         if (np == nullptr) c.misses += 1;
-        if (np) utils::atomic_store(static_cast<uint64_t*>(np), (uint64_t)m_slot[i]);
-        utils::atomic_store(&ptrs[m_slot[i]],
+        if (np) utils::atomic_store(static_cast<uint64_t*>(np), (uint64_t)m_slot[threadIdx.x]);
+        utils::atomic_store(&ptrs[m_slot[threadIdx.x]],
                             np ? reinterpret_cast<uint64_t>(np) : kMallocFailed);
       }
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -708,7 +698,14 @@ unsigned batch_grid(K kernel, int threads, uint64_t chunks, uint32_t workgroups)
 }
 
 constexpr uint32_t kStreamSpinCap = 1u << 22;  // polls of a free waiting for its entry
-constexpr int kRunOps = 1024;  // largest batch of a run of per-thread batches
+// Largest batch of a run of per-thread batches.  With more mallocs the run
+// loses to a launch of its own, which spreads them over more CUs: lognormal
+// sizes, us per batch of 256, 512, 640 and 768 ops in a run / in launches,
+// batches of mallocs and batches of frees in turn 10.3 / 13.8, 13.9 / 15.4,
+// 15.2 / 15.9, 16.8 / 16.1, mallocs and frees mixed 60 : 40 12.4 / 19.4, 15.9 /
+// 21.9, 18.0 / 23.0, 19.3 / 22.9.
+constexpr uint32_t kRunOps = 640;
+constexpr int kRunThreads = kRunOps + 64;  // of such a run (k_run_plain)
 
 template <int kThreads>
 void launch_batched(gal_state* s, const gal_batch_op* ops, uint64_t n, uint64_t* ptrs,
@@ -823,7 +820,8 @@ static int enqueue_stream(gal_allocator* a, const gal_batch_op* ops, const uint6
     }
     if (run.nbatches > 1) {
       if (batched == 0)
-        k_run_plain<kRunOps><<<1, kRunOps, 0, st>>>(s, o, run, ptrs, nslots, ctr, kStreamSpinCap);
+        k_run_plain<kRunThreads>
+            <<<1, kRunThreads, 0, st>>>(s, o, run, ptrs, nslots, ctr, kStreamSpinCap);
       else if (threads == 256)
         k_run_batched<256><<<1, 256, 0, st>>>(s, o, run, ptrs, nslots, ctr, kStreamSpinCap);
       else if (threads == 512)

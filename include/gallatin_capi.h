@@ -438,16 +438,15 @@ int gal_serving_destroy(gal_serving *s);
  * slot >= nslots or an unknown kind also counts there and is skipped).  A
  * batch may free a slot and fill it again in a later op.  A free whose entry
  * was never filled, and a malloc into an entry that nothing frees, wait for a
- * bounded time and count in counter [5].  One
- * persistent launch per batch (with batched 0 or 1, consecutive batches of at
- * most 1024 or `threads` ops share one, in order), then one launch freeing
- * whatever is left in ptrs[0 .. nslots), so the table is empty again at the
- * end.  batched: 0
- * plain per-thread malloc/free; 1 the workgroup-batched path (batched.hpp);
- * 2 mallocs through each workgroup's LDS slice cache (slice_cache.hpp) and
- * per-wave frees.  threads: 256, 512 or 1024 (0 = 1024; modes 1 and 2
- * only); workgroups: 0 = fill the device.  Counters as for the workload
- * kernels. */
+ * bounded time and count in counter [5].  One persistent launch per batch,
+ * then one launch freeing whatever is left in ptrs[0 .. nslots), so the table
+ * is empty again at the end.  With batched 0 or 1, consecutive batches of at
+ * most 640 or `threads` ops share a launch of one workgroup, in order.
+ * batched: 0 plain per-thread malloc/free; 1 the workgroup-batched path
+ * (batched.hpp); 2 mallocs through each workgroup's LDS slice cache
+ * (slice_cache.hpp) and per-wave frees.  threads: 256, 512 or 1024 (0 = 1024;
+ * modes 1 and 2 only); workgroups: at most this many per launch, 0 = fill the
+ * device.  Counters as for the workload kernels. */
 typedef struct gal_batch_op {
   uint64_t arg;   /* malloc: bytes */
   uint32_t kind;  /* 0 malloc, 1 free */

@@ -84,7 +84,7 @@ __global__ void k_boot(gal_state* s) {
     const uint32_t per = s->slot_count[t] / s->num_parts;
     for (uint32_t i = 0; i < s->slot_count[t]; ++i) {
       bool emptied;
-      const uint32_t blk = wave::readfirst(detail::request_new_blocks(
+      const uint32_t blk = wave::readfirst(detail::request_new_blocks<false>(
           s, t, i / per, true, s->lim_request, wave::is_first(), emptied));
       if (__ballot(emptied)) detail::prefetch_segment(s, t, i / per);
       if (blk == kNullBlock) {

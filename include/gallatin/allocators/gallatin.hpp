@@ -388,13 +388,15 @@ __device__ inline void retire_block(gal_state* s, uint32_t blk, uint32_t my_p) {
 // and adding back, held up those that did.  malloc of 64 KiB blocks on 8
 // partitions, 256 threads per workgroup: 4,000 147 -> 59 us, 16,384 890 -> 134
 // us, 30,000 2,210 -> 220 us (one request after another: 406, 490, 658 us).
+// kMany = false: this lane alone.
+template <bool kMany>
 __device__ inline uint64_t get_blocks(gal_state* s, uint64_t seg, uint32_t t, uint32_t p,
                                       bool look, uint64_t group) {
-  const int leader = wave::first(group);
-  const uint32_t rank = wave::count(group & wave::lanes_below());
+  const int leader = kMany ? wave::first(group) : 0;
+  const uint32_t rank = kMany ? wave::count(group & wave::lanes_below()) : 0;
   uint32_t got = 0, q = 0, last = 0;
-  if ((int)wave::lane() == leader) {
-    uint32_t want = wave::count(group);
+  if (!kMany || (int)wave::lane() == leader) {
+    uint32_t want = kMany ? wave::count(group) : 1;
     // With `look`, look before taking: a claim subtracts from the count and
     // adds back what it did not find, so with many waves retrying on a segment
     // that has one or two free blocks left every claimer can see the others'
@@ -421,9 +423,11 @@ __device__ inline uint64_t get_blocks(gal_state* s, uint64_t seg, uint32_t t, ui
       }
     }
   }
-  got = wave::fetch(got, leader);
-  q = wave::fetch(q, leader) + rank;
-  last = wave::fetch(last, leader);
+  if (kMany) {
+    got = wave::fetch(got, leader);
+    q = wave::fetch(q, leader) + rank;
+    last = wave::fetch(last, leader);
+  }
   if (rank >= got) return kNullBlock;
   const uint64_t nb = nb_of(s, t);
   uint32_t blk;
@@ -629,6 +633,8 @@ __device__ inline uint64_t find_segment(gal_state* s, uint32_t t, uint32_t p, bo
 // requests of 64 KiB - 2 GiB: 316 us one after another, 178 us together).
 // `emptied`: this lane took its segment's last block, and the caller runs
 // prefetch_segment once it has passed the block on.
+// kMany = false: one lane asks.
+template <bool kMany>
 __device__ inline uint32_t request_new_blocks(gal_state* s, uint32_t t, uint32_t p, bool det,
                                               uint32_t polls, bool want, bool& emptied) {
   int attempts = 0;
@@ -666,7 +672,7 @@ __device__ inline uint32_t request_new_blocks(gal_state* s, uint32_t t, uint32_t
         continue;
       }
       const uint64_t nb = nb_of(s, t);
-      if (!det && k > nb) {
+      if (kMany && !det && k > nb) {
         // the pending lanes take the segments in turn, nb lanes each
         const uint64_t got = gather_new_segments(s, t, p, (uint32_t)((k + nb - 1) / nb));
         const uint64_t have = __ballot(got != kFail);
@@ -688,11 +694,11 @@ __device__ inline uint32_t request_new_blocks(gal_state* s, uint32_t t, uint32_t
     }
     const bool take = want && blk == kNullBlock && seg < kNoSegment;
     const uint64_t group =
-        fresh ? wave::match(__ballot(take), take, seg) : __ballot(take);
+        kMany && fresh ? wave::match(__ballot(take), take, seg) : __ballot(take);
     if (take) {
       // of several lanes on one segment, those past its free blocks would only
       // subtract and add back
-      const uint64_t got = get_blocks(s, seg, t, p, spins > 0 || (k > 1 && !fresh), group);
+      const uint64_t got = get_blocks<kMany>(s, seg, t, p, spins > 0 || (k > 1 && !fresh), group);
       blk = (uint32_t)got;
       if (got >> 32) {
         veb::remove(class_tree(s, t, p), seg);
@@ -732,7 +738,7 @@ __device__ __noinline__ uint32_t refill_slot(gal_state* s, uint32_t t, uint32_t 
   if (cur != kNullBlock) return cur;  // a block, or another wave's refill
   bool emptied;
   const uint32_t nb =
-      request_new_blocks(s, t, p, det, s->lim_request, wave::is_first(), emptied);
+      request_new_blocks<false>(s, t, p, det, s->lim_request, wave::is_first(), emptied);
   release_to_xcd();  // see replace_block
   if (wave::is_first()) {
     atomic_exch(sp, nb);  // the block, or empty again
@@ -761,7 +767,7 @@ __device__ __noinline__ void replace_block(gal_state* s, uint32_t t, uint32_t p,
   if (wave::readfirst(seen) != blk) return;
   bool emptied;
   const uint32_t nb =
-      request_new_blocks(s, t, p, det, s->lim_request, wave::is_first(), emptied);
+      request_new_blocks<false>(s, t, p, det, s->lim_request, wave::is_first(), emptied);
   // The block's counter is cleared before its id can be read from the slot.
   // Waves that still add to the block's last incarnation can hold the
   // clearing exchange back for tens of microseconds; a helper that found the
@@ -901,7 +907,7 @@ __device__ __noinline__ uint64_t malloc_blocks(gal_state* s, bool want, uint32_t
     bool open = (grp >> wave::lane()) & 1;
     for (uint32_t attempt = 0; attempt < s->lim_block && __ballot(open); ++attempt) {
       bool emptied;
-      const uint32_t blk = request_new_blocks(s, t, p, det, polls, open, emptied);
+      const uint32_t blk = request_new_blocks<true>(s, t, p, det, polls, open, emptied);
       if (__ballot(open && blk == kNullBlock)) polls = 1;
       open = open && blk != kNullBlock;
       if (open) {

@@ -67,9 +67,12 @@ struct chaining_block {
     }
   }
 
-  // An empty block, or with `pair` one whose first slot holds (k0, v0).  The
-  // words from the last key on are written one by one where the keys do not
-  // end on 16 bytes.
+  // An empty block.
+  __device__ void init(Key defaultKey) { init(defaultKey, false, Key{}, Val{}); }
+
+  // The same, or with `pair` one whose first slot holds (k0, v0).  The words
+  // from the last key on are written one by one where the keys do not end on
+  // 16 bytes.
   __device__ void init(Key defaultKey, bool pair, Key k0, Val v0) {
     constexpr int kHead = (int)((16 + sizeof(Key) * size) / 16);  // whole 16 bytes of it
     constexpr int kWhole = (kHead * 16 - 16) / (int)sizeof(Key);  // keys in those
@@ -90,7 +93,7 @@ struct chaining_block {
 template <typename table>
 __global__ void chaining_table_fill_buffers(table* t) {
   const uint64_t i = gallatin::utils::get_tid();
-  if (i < t->nblocks) t->attach_block(reinterpret_cast<uint64_t*>(&t->pointer_list[i]), false);
+  if (i < t->nblocks) t->attach_block(reinterpret_cast<uint64_t*>(&t->pointer_list[i]));
 }
 
 template <typename table>
@@ -227,11 +230,17 @@ struct chaining_table {
     return gallatin::hashers::MurmurHash64A(&k, (int)sizeof(Key), seed) % nblocks;
   }
 
-  // chaining_table.cuh:202-219.  Attaches a block at an empty link; with
-  // `pair` it holds (k0, v0).  0: done; otherwise the link is not empty and
-  // its block is returned, or kNoBlock when none could be allocated.
+  // chaining_table.cuh:202-219.  Attaches an empty block at an empty link.
+  // False when no block could be allocated and the link is still empty.
+  __device__ bool attach_block(uint64_t* link) {
+    return attach(link, false, Key{}, Val{}) != kNoBlock;
+  }
+
+  // Attaches a block at an empty link; with `pair` it holds (k0, v0).  0:
+  // done; otherwise the link is not empty and its block is returned, or
+  // kNoBlock when none could be allocated.
   static constexpr uint64_t kNoBlock = 1;
-  __device__ uint64_t attach_block(uint64_t* link, bool pair, Key k0 = Key{}, Val v0 = Val{}) {
+  __device__ uint64_t attach(uint64_t* link, bool pair, Key k0, Val v0) {
     block_type* nb =
         static_cast<block_type*>(gallatin::allocators::global_malloc(sizeof(block_type)));
     if (!nb) {
@@ -253,7 +262,7 @@ struct chaining_table {
     for (uint32_t hop = 0; hop < kMaxHops; ++hop) {
       uint64_t b = ld64(link);
       if (!b) {
-        b = attach_block(link, true, newKey, newVal);
+        b = attach(link, true, newKey, newVal);
         if (!b) return true;
         if (b == kNoBlock) break;
       }

@@ -349,8 +349,10 @@ struct extendible_hash_table {
   //
   // `fresh` = false reads `level` and the entries through the caches: they
   // may be behind, and since the level only grows and entries are only ever
-  // set that only leads to an ancestor of the owner; every caller checks the
-  // bucket's home against its depth and looks again (with fresh = true).
+  // set that only leads to an ancestor of the owner, or to none; every caller
+  // checks the bucket's home against its depth and looks again (with fresh =
+  // true), and where the caches show no entry at all this does.  nullptr: no
+  // bucket.
   // Device-coherent reads of one word from the whole device queue at one
   // memory channel, and scattered ones run at half the rate of cached ones.
   static constexpr int kOwnerFan = 4;
@@ -367,8 +369,13 @@ struct extendible_hash_table {
 #pragma unroll
       for (int j = 0; j < kOwnerFan; ++j)
         if (e[j]) return reinterpret_cast<bucket*>(e[j]);
-      if (top < min_bits + kOwnerFan) return nullptr;
-      top -= kOwnerFan;
+      if (top >= min_bits + kOwnerFan) {
+        top -= kOwnerFan;
+      } else {
+        if (fresh) return nullptr;
+        fresh = true;
+        top = ld(&level);
+      }
     }
   }
 

@@ -467,6 +467,7 @@ struct extendible_hash_table {
         else
           held = try_lock(b, ctl);
       }
+      const bool none = __ballot(held) == 0;  // the wave got no lock this time
       int match, free_slot;
       uint64_t seen;
       scan(held, b, (uint64_t)key, seen, match, free_slot);
@@ -497,12 +498,15 @@ struct extendible_hash_table {
         unlock(b, ctl);
         if (state == 0) b = nullptr;
       } else if (state == 0) {
-        // Locked: the same bucket again a few times, then look up again, which
-        // also keeps the waiting lanes off the word that the holder has to
-        // unlock.  Trying the same bucket until its word shows a split took
-        // 20 ms where this takes 7 (200,000 keys into 16 first buckets);
-        // looking up every time, 1,000 keys in 600 buckets take 56 us, not 50.
-        if (++losses > kSameBucket || !owns(ctl, h)) b = nullptr;
+        // Locked: the same bucket again, and after a few passes in which
+        // another wave kept this one from every lock, look up again: that
+        // keeps the waiting lanes off the word that the holder has to unlock
+        // (trying the same bucket until its word shows a split, 512 inserts of
+        // one key take 3.5 ms, not 1.6).  A lane that only waits for lanes of
+        // its own wave has nobody to make room for, and its look-up would hold
+        // them up: 64 inserts of one key 165 us with look-ups there, now 132;
+        // 256 keys in about 18 buckets 71, now 62; 1,000 keys 54, now 50.
+        if ((none && ++losses > kSameBucket) || !owns(ctl, h)) b = nullptr;
         __builtin_amdgcn_s_sleep(2);
       }
     }

@@ -38,7 +38,9 @@ class Serving:
                                         ctypes.byref(self.handle)))
 
     def step(self, step, arrivals, reserve_segments, p_end, ht_ops, counters, gate=0):
-        """gate 0: admit while the segment tree has more than reserve_segments
+        """p_end, the chance of a session to end in the step, is below 1: it
+        is passed as 32 bits of fraction, and 1.0 wraps to 0 (none ends).
+        gate 0: admit while the segment tree has more than reserve_segments
         free segments; gate 1: while the free memory (free segments plus the
         free blocks of formatted segments, in segments) exceeds it."""
         _check(lib().gal_serving_step(self.handle, step, arrivals, reserve_segments, gate,

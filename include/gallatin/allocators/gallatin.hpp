@@ -11,9 +11,12 @@
 //  * every entry point is called by the active lanes of a wave together; the
 //    lanes are partitioned by size class (malloc) or block (free) with
 //    ballots, every group's counter atomic is issued in one instruction by
-//    the group leaders, and the rare paths (block turnover, segment setup and
-//    release, whole-block and multi-segment requests) run one request at a
-//    time in lane order with the whole wave available for tree searches;
+//    the group leaders, and the rare paths share their tree searches, which
+//    use the whole wave: whole-block requests of a class are served together,
+//    multi-segment runs and emptied blocks are freed side by side, and
+//    multi-segment requests are carved from one claim where they fit.  In the
+//    deterministic mode these run one at a time in lane order, as the
+//    refills of pinned slots always do;
 //  * tree searches scan 64 words per pass across the wave (veb.hpp);
 //  * the pinned slots and class trees are split into partitions, one per
 //    XCD.  A formatted segment has a home partition; only waves of that XCD
@@ -203,7 +206,7 @@ __device__ inline void clear_chunk_id(gal_state* s, uint64_t seg) {
 // ----------------------------------------------------------- per lane ops
 
 // Ring tickets [f, f + k) of segment seg have just been completed: their k
-// blocks become available to get_block, and the segment goes back to its
+// blocks become available to get_blocks, and the segment goes back to its
 // class tree or, when every block is back, to the segment tree
 // (gallatin.cuh:1646-1722, memory_table.cuh:1226-1241).
 __device__ inline void complete_run(gal_state* s, uint64_t seg, uint32_t t, uint32_t h,
@@ -493,8 +496,10 @@ __device__ inline uint64_t pinned_block(const gal_state* s, uint32_t t, uint32_t
 }
 
 // --------------------------------------------------------- wave ops
-// Functions below are called with identical arguments on every active lane
-// and return wave-uniform results.
+// Functions below are called by the active lanes of a wave together, with
+// identical arguments and wave-uniform results.  gather_new_segments,
+// request_new_blocks and malloc_blocks also take or return a value per lane:
+// their `want`, their result and `emptied`.
 
 __device__ __forceinline__ bool try_lock(gal_state* s, uint32_t idx) {
   uint32_t got = 0;

@@ -12,8 +12,8 @@
 //     of w words is scanned by the wave 64 words per pass;
 //   * the per-segment chunk id (u16) and active count (int) are packed into
 //     one 64-bit word `seg_state` = (active << 32) | tree_id, so `free` reads
-//     one aligned word per pointer and `get_block` learns count and owner in
-//     one atomic;
+//     one aligned word per pointer and `get_blocks` learns count and owner
+//     in one atomic;
 //   * ring entries and pinned slots hold 32-bit block ids instead of Block*.
 #ifndef GALLATIN_LAYOUT_HPP
 #define GALLATIN_LAYOUT_HPP

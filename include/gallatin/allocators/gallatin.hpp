@@ -698,10 +698,8 @@ __device__ inline uint32_t request_new_blocks(gal_state* s, uint32_t t, uint32_t
       }
     }
     const bool take = want && blk == kNullBlock && seg < kNoSegment;
-    // the lanes on this lane's segment; fresh ones of one block have one each
-    uint64_t group = __ballot(take);
-    if (kMany && fresh)
-      group = nb_of(s, t) == 1 ? 1ULL << wave::lane() : wave::match(group, take, seg);
+    const uint64_t group =
+        kMany && fresh ? wave::match(__ballot(take), take, seg) : __ballot(take);
     if (take) {
       // of several lanes on one segment, those past its free blocks would only
       // subtract and add back

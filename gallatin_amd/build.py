@@ -104,6 +104,49 @@ def parse_resource_usage(text):
     return out
 
 
+def assembly(src, out):
+    """Device assembly of one source, compiled as build_hip compiles it."""
+    _run([_hipcc(), *HIP_FLAGS, "-w", "-I", INCLUDE, "-I", os.path.join(HERE, "csrc"),
+          "--cuda-device-only", "-S", src, "-o", out], False)
+    with open(out) as f:
+        return f.read()
+
+
+def shift_hazards(text):
+    """(kernel, function, register) for every 64-bit shift by the last vector
+    register of a kernel, in device assembly.
+
+    On gfx950 such a shift now and then takes another amount: registers are
+    allocated by eights, and with the amount in the last one of the wave's
+    allocation some waves read a wrong value.  The block queue's enqueue,
+    shifting by its lane number in v119 of 120 registers, gave all 64 lanes of a
+    wave one position in about 6 of 16,384 waves; the same code with 128
+    registers allocated never did.  The compiler does not avoid the form for
+    this target."""
+    bodies = {m.group(1): m.group(2) for m in
+              re.finditer(r"^([\w.$]+):\s*; @\1\n(.*?)^\.Lfunc_end", text, re.M | re.S)}
+    calls, amounts = {}, {}
+    for name, body in bodies.items():
+        calls[name] = {c for c in re.findall(r"([\w.$]+)@(?:rel32|gotpcrel32)@lo", body)
+                       if c in bodies}
+        amounts[name] = {int(r) for r in re.findall(
+            r"v_(?:lshlrev_b64|lshrrev_b64|ashrrev_i64)(?:_e64)? v\[\d+:\d+\], v(\d+),", body)}
+        amounts[name] |= {int(r) for r in re.findall(
+            r"v_lshl_add_u64 v\[\d+:\d+\], [^,]+, v(\d+),", body)}
+    found = []
+    for m in re.finditer(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", text, re.S):
+        used = int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", m.group(2)).group(1))
+        last = (used + 7) // 8 * 8 - 1
+        seen, todo = set(), [m.group(1)]
+        while todo:
+            f = todo.pop()
+            if f in bodies and f not in seen:
+                seen.add(f)
+                todo += calls[f]
+        found += [(m.group(1), f, last) for f in sorted(seen) if last in amounts[f]]
+    return found
+
+
 def build_cpu(verbose=False):
     src = os.path.join(HERE, "csrc", "cpu_baseline.cpp")
     if not os.path.exists(src):
